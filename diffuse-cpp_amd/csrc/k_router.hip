@@ -565,6 +565,50 @@ __global__ __launch_bounds__(RT_THREADS) void k_route(RouteParams rp, RouteBufs 
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         }
+    } else if (nc <= 256) {
+        // one wavefront per token, lane l holding candidates l + 64 r: slot by
+        // slot the wavefront's largest key (a live candidate's is its order
+        // key + 1, a taken one's 0; candidates rise with the expert id, so
+        // ties go to the lowest index).  Every ragged call comes here (no
+        // block routing, all experts).  The phase is a chain of maxima, about
+        // 20 dependent instructions per slot; counting each candidate's rank
+        // over all of them (256 x 256 LDS reads per token) took this kernel
+        // 164.5 us at 77 tokens of 256 experts, top 8, this takes it 10.4.
+        // Past 256 candidates the keys no longer fit four registers per lane.
+        for (int t = wave; t < nt; t += RT_WAVES) {
+            uint32_t k[4];
+            int e[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int c = lane + 64 * r;
+                e[r] = c < nc ? s_cand[c] : 0;
+                k[r] = c >= nc ? 0u : (restrict_cand ? order_key(s_sel[t * E + e[r]]) : s_key[t * E + e[r]]) + 1u;
+            }
+            for (int slot = 0; slot < K; slot++) {
+                uint32_t b = k[0];
+                int br = 0;
+#pragma unroll
+                for (int r = 1; r < 4; r++)
+                    if (k[r] > b) {
+                        b = k[r];
+                        br = r;
+                    }
+                const uint32_t top = wave_reduce_u32<true>(b);
+                uint64_t m = __ballot(b == top);
+                if (__popcll(m) > 1) {
+                    const uint32_t c = b == top ? (uint32_t)(lane + 64 * br) : ~0u;
+                    m = __ballot(c == wave_reduce_u32<false>(c));
+                }
+                if (lane == __builtin_ctzll(m)) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (r == br) {
+                            s_idx[t * K + slot] = e[r];
+                            k[r] = 0u;
+                        }
+                }
+            }
+        }
     } else {
         // keys: the sel' keys, or with restricted candidates the keys of sel
         auto key = [&](int t, int e) -> uint32_t {
