@@ -357,9 +357,10 @@ bool use_gemm_path(const dmoe_hparams &hp, int32_t wtype, int32_t stype, bool sh
 // The Q4_K grouped GEMM of k_expert_gemm.hip (units of up to 128 pairs, each
 // step's weight tiles applied to all of a unit's pairs): by the forward's
 // pairs per expert averaged over all experts, N k / E of at least
-// GEMM_Q4K_MIN_AVG.  DMOE_EXPERT_GEMM = 0 / 1 turns it off / on for every N;
+// GEMM_Q4K_MIN_AVG (the flash layer: 1,024 tokens 597 us against 635 on the tile kernels, 512
+// tokens 394 against 386, 256 tokens 284 against 264).  DMOE_EXPERT_GEMM = 0 / 1 turns it off / on for every N;
 // DMOE_EXPERT_TILE or DMOE_Q4K_COLUMN_BLOCKS set selects their kernels.
-constexpr long GEMM_Q4K_MIN_AVG = 64;
+constexpr long GEMM_Q4K_MIN_AVG = 32;
 
 bool use_q4k_gemm(const KernelSwitches &sw, const dmoe_hparams &hp, int32_t wtype, int32_t stype, bool shared,
                   int N)
@@ -492,6 +493,7 @@ size_t plan_workspace(const KernelSwitches &sw, const dmoe_hparams &hp, int32_t 
                  : tile                                         ? expert_tile_chunk(wtype)
                  : gemm ? GM
                         : EXPERT_CHUNK * (use_mfma_path(hp, wtype, stype, shared) ? q4k_column_blocks(sw, hp, N) : 1);
+    t.wl.by_size = use_q4k_gemm(sw, hp, wtype, stype, shared, N);
     t.wl.n_ec = (int32_t *)take(4);
     t.wl.ec_expert = (int32_t *)take((size_t)(E + P / EXPERT_CHUNK + 1) * 4);
     t.wl.ec_chunk = (int32_t *)take((size_t)(E + P / EXPERT_CHUNK + 1) * 4);

@@ -18,6 +18,18 @@ __device__ __forceinline__ T ldc(const T *p, int i)
     return ((const __attribute__((address_space(4))) T *)(uintptr_t)p)[i];
 }
 
+// The j-th item of workgroup b of a persistent grid of G workgroups (a
+// multiple of 8) over items in falling order of work: workgroup b takes items
+// k with k % 8 == b % 8 (those of its XCD), one of every G in turn, the
+// workgroups of an XCD in rising and falling order by turns, so that the one
+// that took a round's largest item takes the next round's smallest.  An item
+// index never falls below an earlier round's.
+__device__ __forceinline__ int schedule_item(int b, int G, int j)
+{
+    const int g8 = G >> 3, i = b >> 3;
+    return 8 * (j * g8 + ((j & 1) ? g8 - 1 - i : i)) + (b & 7);
+}
+
 // The f32 epilogue of one Q4_K super-block product: acc + dx (d S - dmin M),
 // rounded the same way in every kernel whatever its file's contraction
 // setting: d S rounded, then two fused multiply-adds.  (Left to

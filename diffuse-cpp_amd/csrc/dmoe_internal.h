@@ -63,9 +63,13 @@ struct RouteBufs {
 constexpr int ROUTE_LDS = 8192;
 
 // Work list of the expert kernels: one entry per (expert, chunk of `chunk`
-// consecutive pairs of that expert), in expert order.
+// consecutive pairs of that expert), in expert order, or (by_size) the whole
+// chunks first and the experts' remainders after them by falling size, for
+// the kernels that deal the entries out to their workgroups (schedule_item).
+// The order is a matter of speed alone.
 struct WorkList {
     int32_t chunk;
+    int32_t by_size;
     int32_t *n_ec;       // [1]
     int32_t *ec_expert;  // [E + N*K/chunk + 1]
     int32_t *ec_chunk;

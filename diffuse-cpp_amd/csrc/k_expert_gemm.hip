@@ -1,32 +1,55 @@
-// k_expert_gemm.hip — Q4_K expert products as a grouped int8-MFMA GEMM when
-// many pairs reach each expert (prompt prefill and the sampler's large
-// windows, N = 32 (blk + 1) of a thousand tokens and more):
+// k_expert_gemm.hip — Q4_K products as a grouped int8-MFMA GEMM when many rows
+// share each weight (prompt prefill and the sampler's large windows,
+// N = 32 (blk + 1) of a thousand tokens and more):
 // src/diffuse-moe-graph.cpp:264-269 (ggml's mul_mat_id over Q4_K weights
-// with Q8_K activations) and the shared expert of :280-286 (F32 activations
-// as two int8 digits).
+// with Q8_K activations), the shared expert of :280-286 (F32 activations
+// as two int8 digits) and, with shared units only, projections of more than a
+// few tokens.
 //
-// Units: work-list entries of up to 128 pairs of one expert (eight column
-// blocks of 16) and chunks of 64 tokens of the shared expert (their a1 / a0
-// digit rows interleaved, eight blocks of 16 rows).  Items: (unit, row
-// group); gate/up items hold 128 h rows (wavefront w: the gate and the up
-// tile of rows 16 w .. + 15), down items 256 n_embd rows (wavefront w: rows
-// 32 w .. + 31, two tiles).  Workgroup b of G (one per CU, G a multiple of
-// 8) runs items b, b + G, b + 2 G, ...: with row groups a multiple of 8 per
-// unit, one row group of every unit runs on one XCD (workgroup b is placed
-// on XCD b % 8) and consecutive units together, so the chunks of one expert
-// read its weights once from HBM and then from that XCD's L2.
+// Units: work-list entries of up to 128 pairs of one expert (eight 16-row
+// blocks) and chunks of 64 tokens of the shared expert (two int8 digit rows
+// each, eight blocks again).  Items: (unit, row group); an item is 256 weight
+// rows, 32 per wavefront: gate/up items 128 h rows (wavefront w: the gate and
+// the up tile of rows 16 w .. + 15), down items 256 n_embd rows (wavefront
+// w: rows 32 w .. + 31).  One workgroup per CU walks its items
+// (schedule_item): with row groups a multiple of 8 per unit, one row group of
+// every unit runs on one XCD (workgroup b is placed on XCD b % 8) and
+// consecutive units together, so chunks of one expert next to each other read
+// its weights once from HBM and then from that XCD's L2.  The units go out by
+// falling size, the shared ones first, then the work list (by_size): at 2,048
+// tokens a CU runs about seven units of one to eight blocks, and in expert
+// order a wavefront was busy for 0.76 (gate/up) of the launch.
 //
-// Pipeline: one step per 256-value super-block of the reduction.  The
-// step's 16 weight tiles (36 KB, each a 2304-byte run of the tiled layout)
-// and its 128 activation rows (eight 4672-byte blocks) go to one LDS stage
-// by LDS-direct loads, two stages, the next step's loads issued before the
-// current step is computed and continuing across items.  A CU returns
-// vector-memory data in issue order, so the weights and the activations of
-// a step travel together.  Each wavefront folds its two tiles' sub-block
-// scales into the int8 weight operands once per step (compute_folded's
-// sh / sl split) and applies them to all eight blocks: per byte brought into
-// the CU an item does 2.5 times the int8 products of a 32-pair unit of the
-// tile kernels (k_expert_tile.hip), whose launches are bound by that intake.
+// Pipeline: one step per 256-value super-block of the reduction.  A
+// wavefront's 32 weight rows are private to it: one LDS buffer of their own
+// (the tiled layout's runs as they lie), read to registers at the start of a
+// step and refilled for the next step right after, so it needs no second
+// stage.  The step's 128 activation rows lie in a ring of three stages shared
+// by the workgroup, filled two steps ahead.  Both by LDS-direct loads, across
+// items; the waits count the loads issued since, so the younger activation
+// stage stays in flight.
+//
+// Products: v_mfma_i32_32x32x32_i8 on 32 activation rows x 32 weight rows.
+// The sub-block scales are folded into the int8 weight operand once per step
+// (sc = 8 sh + sl, sh and sl below 8: sh q and sl q are int8) and applied to
+// all the unit's rows.  What bounds a step is the SIMD's issue and, in steady
+// state, the power that issue takes: per 32 x 32 output tile and super-block 16
+// int8 MFMAs of 32 cycles (twice the useful products: the two scale digits; 44
+// cycles each in steady state on such operands), 80 VALU instructions of scale
+// epilogue (five per output) and the fold's ~150 shared by up to four tiles.
+// Launches with shared units only (MERGE) keep a token's two digit rows in
+// separate blocks of 32, so that both digits of an output lie in one lane and
+// take one epilogue (8 instructions per token against 10).
+//
+// Measured (steady state, the card at its power limit, against 16 x 16 MFMA
+// tiles with one epilogue per digit row, the weights and activations of a step
+// in one of two shared stages, units in expert order): Q4_K MoE layer of 2,048
+// tokens 1,073 -> 1,012 us, of 1,024 tokens 646 -> 582; dense MLP of 160 tokens
+// 129 -> 110 us, of 512 314 -> 286; attention half of 777 tokens 268 -> 247, of
+// 2,048 612 -> 603 us.  In bursts too short to reach the power limit the MoE
+// launches gain more (620 -> 497 and 314 -> 300 us at 2,048 tokens, mostly the
+// schedule); in steady state an even schedule buys less, since busy CUs run
+// faster while others wait.
 //
 // Arithmetic: the integer sums of every super-block are compute_sb's exactly
 // (8 sum (sh q) a + sum (sl q) a = sum_j sc_j S_j), then one f32 epilogue per
@@ -37,26 +60,45 @@
 // ys [token][n_embd] for the combine launch, as with the tile kernels.
 #include "dmoe_q4k.h"
 
+#include <type_traits>
+
 namespace dmoe {
 
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+
 constexpr int XG_WAVES = 8;
-constexpr int XG_NC = 8;                                     // column blocks of a unit
+constexpr int XG_NC = 8;                                     // 16-row blocks of a unit
 constexpr int XG_CHUNK = EXPERT_CHUNK * XG_NC;               // routed pairs of a unit (128)
 constexpr int XG_SCHUNK = SHARED_CHUNK * XG_NC;              // shared tokens of a unit (64)
 constexpr int XG_GU_ROWS = XG_WAVES * 16;                    // h rows of a gate/up item
 constexpr int XG_DN_ROWS = XG_WAVES * 32;                    // n_embd rows of a down item
-constexpr int XG_WBYTES = XG_WAVES * 2 * TILE_BYTES;         // weights of a stage (36,864)
-constexpr int XG_STAGE = XG_WBYTES + XG_NC * ASTEP_BYTES;    // 74,240
-static_assert(XG_STAGE % 16 == 0 && TILE_BYTES % 16 == 0 && ASTEP_BYTES % 16 == 0, "16-byte pieces");
-static_assert(TPIECES > 128 && TPIECES <= 144, "a tile is two 64-lane loads and one of 16 lanes");
 
-// Item k is row group k % rg_n of unit k / rg_n; a unit is work-list entry
-// u < n_ec, else shared chunk u - n_ec.  Every field is wave-uniform.
+// A stage of the activation ring: four blocks of 32 rows.  A block's int8
+// values lie in eight chunks of four rows (1 KB each, as one LDS-direct load
+// writes them): row r of the block at 1024 (r / 4) + 64 (r / 8) + 256 (r % 4),
+// its 16-byte unit 8 gp + 4 h + c (values as the ActI8 layout orders them) at
+// slot 8 gp + 4 h + (c ^ (r % 4)).  An operand read (lane: row l % 32, h =
+// l / 32, one (gp, c)) takes four rows' units from 64 bytes of each chunk, and
+// the 64-byte step between chunk pairs puts the four lane quads that are
+// served together on different banks.  Then the 32 rows' sums of 16 (f16) and
+// scales.
+constexpr int XG_ABS = 8 * 1024 + 3 * 64;                    // sums of 16: [32][16] f16
+constexpr int XG_AD = XG_ABS + 1024;                         // scales: [32] f32
+constexpr int XG_ABLK = XG_AD + 128;                         // one block (9,344)
+constexpr int XG_ASTAGE = (XG_NC / 2) * XG_ABLK;
+constexpr int XG_AHEAD = 4;                                  // operand reads ahead of their MFMAs (divides 8)
+static_assert(XG_ABLK % 16 == 0, "16-byte pieces");
+
+// Item k is row group k % rg_n of unit k / rg_n; a unit is shared chunk
+// u < nch, else work-list entry u - nch.  Every field is wave-uniform.
 struct XgItem {
     int rg, e, t_first, nt, nblk;
     bool shared, valid;
 };
 
+template <bool MERGE>
 __device__ __forceinline__ XgItem xg_decode(const MoeJob &job, int k, int rg_n, int n_ec, int nch)
 {
     XgItem I{};
@@ -64,29 +106,39 @@ __device__ __forceinline__ XgItem xg_decode(const MoeJob &job, int k, int rg_n, 
     I.rg = k - unit * rg_n;
     I.valid = unit < n_ec + nch;
     if (!I.valid) return I;
-    I.shared = unit >= n_ec;
+    I.shared = unit < nch;
     if (!I.shared) {
-        I.e = ldc(job.wl.ec_expert, unit);
-        const int c0 = ldc(job.wl.ec_chunk, unit) * XG_CHUNK;
+        I.e = ldc(job.wl.ec_expert, unit - nch);
+        const int c0 = ldc(job.wl.ec_chunk, unit - nch) * XG_CHUNK;
         I.t_first = ldc(job.offsets, I.e) + c0;
         I.nt = min(XG_CHUNK, ldc(job.counts, I.e) - c0);
         I.nblk = (I.nt + EXPERT_CHUNK - 1) / EXPERT_CHUNK;
     } else {
         I.e = 0;
-        I.t_first = (unit - n_ec) * XG_SCHUNK;
+        I.t_first = unit * XG_SCHUNK;
         I.nt = min(XG_SCHUNK, job.n_tokens - I.t_first);
-        I.nblk = (I.nt + SHARED_CHUNK - 1) / SHARED_CHUNK;
+        // MERGE: 32-token blocks (four 16-row blocks), the last one a half
+        // block (two) when it holds up to 16 tokens
+        I.nblk = MERGE ? 2 * ((I.nt + 15) / 16) : (I.nt + SHARED_CHUNK - 1) / SHARED_CHUNK;
     }
     return I;
 }
 
-// Activation row of block row r (0..15) of block c: routed rows from the
+// Activation row of row r (0..15) of 16-row block c: routed rows from the
 // item's pair ids (x by token, pid / K, for gate/up; h by pair for down);
-// shared items interleave the a1 / a0 digit rows (a0 rows start at N).
-// Rows past the item's last repeat it.
-template <bool DOWN>
+// shared items interleave the a1 / a0 digit rows (a0 rows start at N), or
+// (MERGE) hold the a1 rows of 32 tokens in blocks 4 b, 4 b + 1 and their a0
+// rows in blocks 4 b + 2, 4 b + 3, a last half block of up to 16 tokens the a1
+// rows in block 4 b and the a0 rows in 4 b + 1.  Rows past the item's last
+// repeat it.
+template <bool DOWN, bool MERGE>
 __device__ __forceinline__ int xg_arow(const XgItem &I, const int32_t *s_pids, int N, int K, int c, int r)
 {
+    if (MERGE) {
+        const bool half = (c | 3) >= I.nblk;
+        const int t = 32 * (c >> 2) + (half ? 0 : 16 * (c & 1)) + r, a0 = half ? c & 1 : (c >> 1) & 1;
+        return I.t_first + min(t, I.nt - 1) + a0 * N;
+    }
     if (I.shared) return I.t_first + min(SHARED_CHUNK * c + (r >> 1), I.nt - 1) + (r & 1) * N;
     const int p = s_pids[min(EXPERT_CHUNK * c + r, I.nt - 1)];
     return DOWN ? p : p / K;
@@ -116,45 +168,110 @@ __device__ __forceinline__ void xg_lds4(const void *base, uint32_t voff, uint32_
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" : : "v"(voff), "s"(sb), "s"(m0) : "memory", "m0");
 }
 
-// Two folded tiles against one block's activations of the step (the
-// operands read once for both).
-__device__ __forceinline__ void xg_products(const Q4KFolded (&f)[2], const uint8_t *ast, int r16, int g,
-                                            float (&acc)[2][4])
-{
-    const uint4 *ap = reinterpret_cast<const uint4 *>(ast + r16 * 256);
-    v4i a[4];
+// Weight formats.  A lane holds weight row l % 32 (16-row tile (l / 16) % 2 of
+// the wavefront's two) and the values of lane groups g = h and 2 + h (h = l /
+// 32) of a super-block.  Each gives:
+//   TILE, TLDS, WLOADS   bytes of a 16-row tile's super-block in HBM, its
+//                        stride in LDS
+//   ASTAGES, ALOADS      activation stages; loads of a 16-row block
+//   MIN, BASE            a min term on the sums of 16; the two weight digits'
+//                        ratio
+//   Raw, read, pin       the lane's bytes of a super-block, from LDS; in
+//                        registers from there on
+//   Ops, fold            the int8 operands: hi and lo digits of scale x quant,
+//                        chunk c of lane group 2 gp + h at [4 gp + c]
+struct XgQ4K {
+    static constexpr int TILE = TILE_BYTES, TLDS = TILE_BYTES, ASTAGES = 3, ALOADS = 6;
+    static constexpr bool MIN = true;
+    struct Raw {
+        uint4 h, q[4];
+    };
+    // bm: the min-term operand (m of the lane's eight sums of 16: sub-blocks
+    // 4 h .. 4 h + 3, twice each); d, dmin: the row's scales
+    struct Ops {
+        v4i hi[8], lo[8];
+        h8 bm;
+        float d, dmin;
+    };
+    __device__ static void read(Raw &t, const uint8_t *tile, int r16, int h)
+    {
+        const uint4 *p = reinterpret_cast<const uint4 *>(tile);
+        t.h = p[r16];
 #pragma unroll
-    for (int c = 0; c < 4; c++) a[c] = __builtin_bit_cast(v4i, ap[(4 * g + c) ^ (r16 & 11)]);
-    const h4 ab = __builtin_bit_cast(h4, *reinterpret_cast<const uint2 *>(ast + ABS_OFF + r16 * 32 + 8 * g));
-    const float4 dxv = *reinterpret_cast<const float4 *>(ast + AD_OFF + 16 * g);
-    const float dx[4] = {dxv.x, dxv.y, dxv.z, dxv.w};
-#pragma unroll
-    for (int r = 0; r < 2; r++) {
-        v4i sh = {0, 0, 0, 0}, sl = {0, 0, 0, 0};
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[c], f[r].bh[c], sh, 0, 0, 0);
-            sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[c], f[r].bl[c], sl, 0, 0, 0);
-        }
-        f4 s2 = {0.0f, 0.0f, 0.0f, 0.0f};
-        s2 = __builtin_amdgcn_mfma_f32_16x16x16f16(ab, f[r].bm, s2, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int isum = 8 * sh[i] + sl[i];
-            acc[r][i] = q4k_epi(acc[r][i], dx[i], f[r].d, (float)isum, f[r].dmin, s2[i]);
+        for (int gp = 0; gp < 2; gp++) {
+            t.q[2 * gp] = p[(1 + 2 * (2 * gp + h)) * 16 + r16];
+            t.q[2 * gp + 1] = p[(2 + 2 * (2 * gp + h)) * 16 + r16];
         }
     }
-}
+    __device__ static void pin(Raw &t)
+    {
+        asm volatile("" : "+v"(t.h.x), "+v"(t.h.y), "+v"(t.h.z), "+v"(t.h.w));
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            asm volatile("" : "+v"(t.q[i].x), "+v"(t.q[i].y), "+v"(t.q[i].z), "+v"(t.q[i].w));
+    }
+    // sc = 8 sh + sl: hi = sh q, lo = sl q
+    __device__ static void fold(const Raw &t, int h, Ops &f)
+    {
+        typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+        // scale j: 6 bits at 6j of dword y (j < 5), at 6 (j - 5) of dword z
+        uint32_t sh[8], sl[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const uint32_t src = j < 5 ? t.h.y : t.h.z;
+            const uint32_t off = j < 5 ? 6u * j : 6u * (j - 5);
+            sl[j] = bfe(src, off, 3);
+            sh[j] = bfe(src, off + 3, 3);
+        }
+        // byte-wise products by a scale below 8: each byte stays below 128, so
+        // a 16-bit lane product carries nothing across its two bytes
+        auto mul = [](uint32_t v, uint32_t s) -> int {
+            const u16x2 a = __builtin_bit_cast(u16x2, v);
+            const u16x2 b = {(unsigned short)s, (unsigned short)s};
+            return __builtin_bit_cast(int, (u16x2)(a * b));
+        };
+#pragma unroll
+        for (int gp = 0; gp < 2; gp++) {
+            const uint4 q0 = t.q[2 * gp], q1 = t.q[2 * gp + 1];
+            const uint32_t w[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const uint32_t l0 = w[2 * c] & 0x0F0F0F0Fu, l1 = w[2 * c + 1] & 0x0F0F0F0Fu;
+                const uint32_t h0 = (w[2 * c] >> 4) & 0x0F0F0F0Fu, h1 = (w[2 * c + 1] >> 4) & 0x0F0F0F0Fu;
+                f.hi[4 * gp + c] =
+                    (v4i){mul(l0, sh[2 * c]), mul(l1, sh[2 * c]), mul(h0, sh[2 * c + 1]), mul(h1, sh[2 * c + 1])};
+                f.lo[4 * gp + c] =
+                    (v4i){mul(l0, sl[2 * c]), mul(l1, sl[2 * c]), mul(h0, sl[2 * c + 1]), mul(h1, sl[2 * c + 1])};
+            }
+        }
+        // mins: m0 m1 at 18, 24 of dword z, m2 .. m6 at 0, 6, .. of dword w, m7 in
+        // bits 30..31 of the three dwords
+        const uint32_t m7 = (t.h.y >> 30) | ((t.h.z >> 30) << 2) | ((t.h.w >> 30) << 4);
+        const uint32_t mm[4] = {h ? bfe(t.h.w, 12, 6) : bfe(t.h.z, 18, 6), h ? bfe(t.h.w, 18, 6) : bfe(t.h.z, 24, 6),
+                                h ? bfe(t.h.w, 24, 6) : bfe(t.h.w, 0, 6), h ? m7 : bfe(t.h.w, 6, 6)};
+#pragma unroll
+        for (int i = 0; i < 4; i++) f.bm[2 * i] = f.bm[2 * i + 1] = (_Float16)(float)mm[i];
+        f.d = h16f(t.h.x & 0xffffu);
+        f.dmin = h16f(t.h.x >> 16);
+        // (as an f32 operand: folded into v_fma_mix_f32 the epilogue's min term
+        // issues at half the rate of v_fmac_f32)
+        asm volatile("" : "+v"(f.dmin));
+    }
+};
 
-template <bool DOWN>
-__global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q4k(MoeJob job)
+template <class F, bool DOWN, bool MERGE>
+__global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
 {
-    __shared__ __align__(16) uint8_t S[2][XG_STAGE];
-    __shared__ int32_t s_pids[2][XG_CHUNK];          // routed items: their pair ids
+    constexpr int NBMAX = MERGE ? XG_NC / 4 : XG_NC / 2;   // 32-row (MERGE: 32-token) blocks of a unit
+    __shared__ __align__(16) uint8_t SA[F::ASTAGES][XG_ASTAGE];
+    __shared__ __align__(16) uint8_t SW[XG_WAVES][2 * F::TLDS];
+    // pair ids of the routed items i, i + 1 (its activations load during
+    // item i) and i + 2 (read from perm during item i, written at its end)
+    __shared__ int32_t s_pids[3][XG_CHUNK];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int g = lane >> 4, r16 = lane & 15;
+    const int r16 = lane & 15, r32 = lane & 31, h = lane >> 5;
     const int H = job.H, FF = job.FF, N = job.n_tokens, K = job.top_k;
     const int n_ec = job.wl.n_ec ? ldc(job.wl.n_ec, 0) : 0;   // none: shared units only
     const int nch = job.has_shared ? (N + XG_SCHUNK - 1) / XG_SCHUNK : 0;
@@ -163,187 +280,411 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q4k(MoeJob job)
     // down launches of a projection split the reduction into KS slices of
     // `steps` super-blocks (item k: slice k % KS of item k / KS)
     const int KS = DOWN && job.ks > 1 ? job.ks : 1;
-    const int steps = Kin / 256 / KS;                // >= 2
+    const int nsb = Kin / 256, steps = nsb / KS;     // >= 2
     const int G = gridDim.x;
 
-    int k = blockIdx.x;
-    XgItem I = xg_decode(job, k / KS, rg_n, n_ec, nch);
+    int k = schedule_item(blockIdx.x, G, 0), round = 0;
+    XgItem I = xg_decode<MERGE>(job, k / KS, rg_n, n_ec, nch);
     if (!I.valid) return;
     int slice = k % KS;
-    XgItem NI = xg_decode(job, (k + G) / KS, rg_n, n_ec, nch);
-    int nslice = (k + G) % KS;
+    k = schedule_item(blockIdx.x, G, 1);
+    XgItem NI = xg_decode<MERGE>(job, k / KS, rg_n, n_ec, nch);
+    int nslice = k % KS;
     if (tid < XG_CHUNK && !I.shared) s_pids[0][tid] = job.perm[I.t_first + min(tid, I.nt - 1)];
+    if (tid < XG_CHUNK && NI.valid && !NI.shared) s_pids[1][tid] = job.perm[NI.t_first + min(tid, NI.nt - 1)];
     __syncthreads();
 
-    // The load cursor (one step ahead of the products, across items): this
-    // wavefront's two weight tiles and, for wavefront w < the cursor item's
-    // blocks, block w's activation arrays (wave-uniform bases) and this
-    // lane's byte offsets into them (32-bit: the host keeps every activation
-    // array below 2 GiB).
+    // Load cursors, across items: the weights run one step ahead of the
+    // products, the activations two.  Wave-uniform bases; wavefront w loads
+    // 16-row block w of the items that have it, by this lane's byte offsets
+    // (32-bit: the host keeps every activation array below 2 GiB).
+    const uint32_t sw = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)&SW[wave][0];
+    const uint32_t sa = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)&SA[0][0];
     const uint8_t *wb0 = nullptr, *wb1 = nullptr;
     const uint8_t *aqb = nullptr, *absb = nullptr, *adb = nullptr;
     uint32_t aqo[4] = {0, 0, 0, 0}, abso = 0, ado = 0;
     bool act_on = false;
-    // (the cursor's slice cs starts at super-block cs * steps of every row)
-    auto set_cursor = [&](const XgItem &C, int cs, const int32_t *pids) {
-        const int nsb = Kin / 256, sb0 = cs * steps;
+    // (slice cs of an item starts at super-block cs * steps of every row)
+    auto weights_of = [&](const XgItem &C, int cs) {
         if (!DOWN) {
             const WTensor &a = C.shared ? job.sg : job.eg;
             const WTensor &b = C.shared ? job.su : job.eu;
             const int t16 = C.rg * (XG_GU_ROWS / 16) + wave;
-            wb0 = a.data + (size_t)C.e * a.nb2 + (size_t)t16 * nsb * TILE_BYTES;
-            wb1 = b.data + (size_t)C.e * b.nb2 + (size_t)t16 * nsb * TILE_BYTES;
+            wb0 = a.data + (size_t)C.e * a.nb2 + (size_t)t16 * nsb * F::TILE;
+            wb1 = b.data + (size_t)C.e * b.nb2 + (size_t)t16 * nsb * F::TILE;
         } else {
             const WTensor &W = C.shared ? job.sd : job.ed;
             const int t16 = C.rg * (XG_DN_ROWS / 16) + 2 * wave;
-            wb0 = W.data + (size_t)C.e * W.nb2 + ((size_t)t16 * nsb + sb0) * TILE_BYTES;
-            wb1 = wb0 + (size_t)nsb * TILE_BYTES;
+            wb0 = W.data + (size_t)C.e * W.nb2 + ((size_t)t16 * nsb + cs * steps) * F::TILE;
+            wb1 = wb0 + (size_t)nsb * F::TILE;
         }
+    };
+    auto acts_of = [&](const XgItem &C, int cs, const int32_t *pids) {
         act_on = wave < C.nblk;
-        if (act_on) {
-            const ActI8 &A = DOWN ? (C.shared ? job.ahs : job.ah) : (C.shared ? job.axs : job.ax);
-            aqb = reinterpret_cast<const uint8_t *>(A.q) + (size_t)sb0 * 256;
-            absb = reinterpret_cast<const uint8_t *>(A.bs) + (size_t)sb0 * 32;
-            adb = reinterpret_cast<const uint8_t *>(A.d) + (size_t)sb0 * 4;
+        if (!act_on) return;
+        const int sb0 = cs * steps;
+        const ActI8 &A = DOWN ? (C.shared ? job.ahs : job.ah) : (C.shared ? job.axs : job.ax);
+        aqb = reinterpret_cast<const uint8_t *>(A.q) + (size_t)sb0 * 256;
+        absb = reinterpret_cast<const uint8_t *>(A.bs) + (size_t)sb0 * 32;
+        adb = reinterpret_cast<const uint8_t *>(A.d) + (size_t)sb0 * 4;
+        // (the lane through an empty asm: its rows and units are formed here,
+        // once per item, and not held in registers across the steps)
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int u = ((ln & 15) ^ (ln >> 4)) * 16;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int r = 4 * j + (lane >> 4);
-                aqo[j] = (uint32_t)xg_arow<DOWN>(C, pids, N, K, wave, r) * (uint32_t)Kin + (((lane & 15) ^ (r & 11)) * 16);
-            }
-            abso = ((uint32_t)xg_arow<DOWN>(C, pids, N, K, wave, (lane >> 1) & 15) * (uint32_t)(Kin / 16) + (lane & 1) * 8) * 2;
-            ado = (uint32_t)xg_arow<DOWN>(C, pids, N, K, wave, lane & 15) * (uint32_t)(Kin / 256) * 4;
-        }
+        for (int j = 0; j < 4; j++)
+            aqo[j] = (uint32_t)xg_arow<DOWN, MERGE>(C, pids, N, K, wave, 4 * j + (ln >> 4)) * (uint32_t)Kin + u;
+        abso = ((uint32_t)xg_arow<DOWN, MERGE>(C, pids, N, K, wave, (ln >> 1) & 15) * (uint32_t)(Kin / 16) + (ln & 1) * 8) * 2;
+        ado = (uint32_t)xg_arow<DOWN, MERGE>(C, pids, N, K, wave, ln & 15) * (uint32_t)(Kin / 256) * 4;
     };
-    // the cursor's super-block sb into stage st (LDS addresses as 32-bit
-    // offsets of the LDS aperture)
-    const uint32_t s_lds = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)&S[0][0];
-    auto issue = [&](int st, int sb) {
-        const uint32_t wd = s_lds + st * XG_STAGE + wave * (2 * TILE_BYTES);
-        const uint8_t *s0 = wb0 + (size_t)sb * TILE_BYTES, *s1 = wb1 + (size_t)sb * TILE_BYTES;
+    // the weight cursor's super-block to the wavefront's buffer; on to the next
+    auto issue_w = [&]() {
+        constexpr int FULL = F::TILE / 1024, REST = (F::TILE % 1024) / 16;
         const uint32_t vo = (uint32_t)lane * 16;
-        xg_lds16(s0, vo, wd);
-        xg_lds16(s0, vo + 1024, wd + 1024);
-        xg_lds16(s1, vo, wd + TILE_BYTES);
-        xg_lds16(s1, vo + 1024, wd + TILE_BYTES + 1024);
-        if (lane < TPIECES - 128) {
-            xg_lds16(s0, vo + 2048, wd + 2048);
-            xg_lds16(s1, vo + 2048, wd + TILE_BYTES + 2048);
-        }
-        if (act_on) {
-            const uint32_t ad = s_lds + st * XG_STAGE + XG_WBYTES + wave * ASTEP_BYTES;
-            const uint8_t *qb = aqb + (size_t)sb * 256;
 #pragma unroll
-            for (int j = 0; j < 4; j++) xg_lds16(qb, aqo[j], ad + 1024 * j);
-            if (lane < 32) xg_lds16(absb + (size_t)sb * 32, abso, ad + ABS_OFF);
-            if (lane < 16) xg_lds4(adb + (size_t)sb * 4, ado, ad + AD_OFF);
+        for (int i = 0; i < FULL; i++) {
+            xg_lds16(wb0, vo + 1024 * i, sw + 1024 * i);
+            xg_lds16(wb1, vo + 1024 * i, sw + F::TLDS + 1024 * i);
         }
+        if (lane < REST) {
+            xg_lds16(wb0, vo + 1024 * FULL, sw + 1024 * FULL);
+            xg_lds16(wb1, vo + 1024 * FULL, sw + F::TLDS + 1024 * FULL);
+        }
+        wb0 += F::TILE;
+        wb1 += F::TILE;
     };
+    // the activation cursor's super-block to ring stage st (F::ALOADS loads of
+    // a wavefront that has a block); on to the next
+    auto issue_a = [&](int st) {
+        if (!act_on) return;
+        const uint32_t blk = sa + st * XG_ASTAGE + (wave >> 1) * XG_ABLK;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int q = 4 * (wave & 1) + j;         // chunk of four rows
+            xg_lds16(aqb, aqo[j], blk + 1024 * q + 64 * (q >> 1));
+        }
+        if (F::MIN && lane < 32) xg_lds16(absb, abso, blk + XG_ABS + 512 * (wave & 1));
+        if (lane < 16) xg_lds4(adb, ado, blk + XG_AD + 64 * (wave & 1));
+        aqb += 256;
+        absb += 32;
+        adb += 4;
+    };
+    // this lane's operand addresses in a stage: row r32, unit 8 gp + 4 h + c
+    // (c's swizzle in the address, gp 128 bytes on)
+    uint32_t ao[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+        ao[c] = 1024 * (r32 >> 2) + 64 * (r32 >> 3) + 256 * (r32 & 3) + 64 * h + 16 * (c ^ (r32 & 3));
+    const uint8_t *wrd = &SW[wave][((lane >> 4) & 1) * F::TLDS];
 
-    set_cursor(I, slice, s_pids[0]);
-    issue(0, 0);
+    weights_of(I, slice);
+    acts_of(I, slice, s_pids[0]);
+    issue_w();
+    issue_a(0);
+    if (F::ASTAGES == 3) issue_a(1);                  // steps >= 2
     int stg = 0;                                      // the stage the products read
-    int buf = 0;                                      // the pair list of item I
-    int npid = 0;                                     // the next item's pair id (tid < 128)
+    bool ahead = act_on;                              // activation loads issued after this step's weights
+    int pb = 0;                                       // pair list of item I (of 3)
 
     for (;;) {
-        float acc[XG_NC][2][4];
-#pragma unroll
-        for (int c = 0; c < XG_NC; c++)
-#pragma unroll
-            for (int r = 0; r < 2; r++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) acc[c][r][i] = 0.0f;
+        const int pb1 = pb == 2 ? 0 : pb + 1, pb2 = pb1 == 2 ? 0 : pb1 + 1;
+        k = schedule_item(blockIdx.x, G, round + 2);
+        const XgItem NNI = xg_decode<MERGE>(job, k / KS, rg_n, n_ec, nch);
+        int npid = 0;
+        if (tid < XG_CHUNK && NNI.valid && !NNI.shared) npid = job.perm[NNI.t_first + min(tid, NNI.nt - 1)];
 
-        for (int s = 0; s < steps; s++) {
-            // the next item's pair list (loaded during step 0) to LDS, then
-            // this step's stage landed in every wavefront and the other stage
-            // read by all of them
-            if (s == 1 && tid < XG_CHUNK) s_pids[buf ^ 1][tid] = npid;
-            EXPERT_WAIT_VM(0);
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            if (s + 1 < steps) {
-                issue(stg ^ 1, s + 1);
-            } else if (NI.valid) {
-                set_cursor(NI, nslice, s_pids[buf ^ 1]);
-                issue(stg ^ 1, 0);
-            }
-            if (s == 0 && tid < XG_CHUNK && NI.valid && !NI.shared)
-                npid = job.perm[NI.t_first + min(tid, NI.nt - 1)];
+        v16f acc[NBMAX];
+#pragma unroll
+        for (int c = 0; c < NBMAX; c++) acc[c] = (v16f)(0.0f);
 
-            const uint8_t *st = S[stg];
-            Q4KFolded f[2];
+        // NB: the item's 32-row (MERGE: 32-token) blocks; HALF: a half block
+        // after them
+        auto run = [&](auto nb_c, auto half_c) __attribute__((always_inline)) {
+            constexpr int NB = decltype(nb_c)::value;
+            constexpr bool HALF = decltype(half_c)::value;
+            for (int s = 0; s < steps; s++) {
+                // this step's weights (this wavefront's) and activations
+                // (every wavefront's) have landed, the stage two steps on has
+                // been read by all
+                if (F::ASTAGES == 3 && ahead)
+                    EXPERT_WAIT_VM(F::ALOADS);
+                else
+                    EXPERT_WAIT_VM(0);
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                typename F::Raw t;
+                F::read(t, wrd, r16, h);
+                F::pin(t);                            // the buffer may be refilled
+                // the stage the activations of step s + LEAD go to
+                constexpr int LEAD = F::ASTAGES - 1;
+                const int st2 = stg == 0 ? LEAD : stg - 1;
+                if (s + 1 < steps) {
+                    issue_w();
+                } else if (NI.valid) {
+                    weights_of(NI, nslice);
+                    issue_w();
+                }
+                if (s + LEAD < steps) {
+                    issue_a(st2);
+                    ahead = act_on;
+                } else if (NI.valid) {
+                    if (s + LEAD == steps) acts_of(NI, nslice, s_pids[pb1]);
+                    issue_a(st2);
+                    ahead = act_on;
+                } else {
+                    ahead = false;
+                }
+                typename F::Ops f;
+                F::fold(t, h, f);
+                // The blocks' products.  The operand reads run XG_AHEAD ahead
+                // of their MFMAs (the next block's first ones go out before
+                // this block's epilogue); the scheduling barriers keep that
+                // order, which the compiler otherwise undoes to save registers.
+                const uint8_t *st = &SA[0][0] + stg * XG_ASTAGE;
+                auto read_a = [&](int b, int i) __attribute__((always_inline)) -> v4i {
+                    return *reinterpret_cast<const v4i *>(st + b * XG_ABLK + ao[i & 3] + 128 * (i >> 2));
+                };
+                if constexpr (MERGE) {
+                    // block c: 32 tokens, their a1 rows in stage block 2 c, a0
+                    // rows in 2 c + 1; the four digit products of a chunk, then
+                    // one epilogue per token
+                    v4i a1[XG_AHEAD / 2], a0[XG_AHEAD / 2];
+                    if (NB)
 #pragma unroll
-            for (int r = 0; r < 2; r++) {
-                Q4KTile t;
-                read_tile(t, st + wave * (2 * TILE_BYTES) + r * TILE_BYTES, r16, g);
-                fold_tile(t, g, f[r]);
+                        for (int i = 0; i < XG_AHEAD / 2; i++) {
+                            a1[i] = read_a(0, i);
+                            a0[i] = read_a(1, i);
+                        }
+#pragma unroll
+                    for (int c = 0; c < NB; c++) {
+                        const uint8_t *ab1 = st + 2 * c * XG_ABLK, *ab0 = ab1 + XG_ABLK;
+                        v16i p11 = (v16i)(0), p10 = (v16i)(0), p01 = (v16i)(0), p00 = (v16i)(0);
+                        v16f s2 = (v16f)(0.0f);
+#pragma unroll
+                        for (int i = 0; i < 8; i++) {
+                            __builtin_amdgcn_sched_barrier(0);
+                            const v4i x1 = a1[i % (XG_AHEAD / 2)], x0 = a0[i % (XG_AHEAD / 2)];
+                            p11 = __builtin_amdgcn_mfma_i32_32x32x32_i8(x1, f.hi[i], p11, 0, 0, 0);
+                            p10 = __builtin_amdgcn_mfma_i32_32x32x32_i8(x1, f.lo[i], p10, 0, 0, 0);
+                            p00 = __builtin_amdgcn_mfma_i32_32x32x32_i8(x0, f.lo[i], p00, 0, 0, 0);
+                            if (F::MIN)
+                                p01 = __builtin_amdgcn_mfma_i32_32x32x32_i8(x0, f.hi[i], p01, 0, 0, 0);
+                            else                      // both weigh 256
+                                p10 = __builtin_amdgcn_mfma_i32_32x32x32_i8(x0, f.hi[i], p10, 0, 0, 0);
+                            const int n = 8 * c + i + XG_AHEAD / 2;
+                            if (n < 8 * NB) {
+                                a1[i % (XG_AHEAD / 2)] = read_a(2 * (n >> 3), n & 7);
+                                a0[i % (XG_AHEAD / 2)] = read_a(2 * (n >> 3) + 1, n & 7);
+                            }
+                            if constexpr (F::MIN)
+                                if (i == 6) {
+                                    // sums of 16: 256 (a1 sums) + (a0 sums), the
+                                    // factor on the operand (m <= 63: exact)
+                                    const h8 s1 = *reinterpret_cast<const h8 *>(ab1 + XG_ABS + r32 * 32 + 16 * h);
+                                    const h8 s0 = *reinterpret_cast<const h8 *>(ab0 + XG_ABS + r32 * 32 + 16 * h);
+                                    s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(s1, f.bm * (_Float16)256.0f, s2, 0, 0, 0);
+                                    s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(s0, f.bm, s2, 0, 0, 0);
+                                }
+                        }
+                        // (the a0 row's scale; the a1 row's is 256 times it)
+                        f4 dx = *reinterpret_cast<const f4 *>(ab0 + XG_AD + 16 * h);
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            f4 nx = dx;
+                            __builtin_amdgcn_sched_barrier(0);
+                            if (j < 3) nx = *reinterpret_cast<const f4 *>(ab0 + XG_AD + 32 * (j + 1) + 16 * h);
+#pragma unroll
+                            for (int k = 0; k < 4; k++) {
+                                const int i = 4 * j + k;
+                                if constexpr (F::MIN) {
+                                    const int t1 = 8 * p11[i] + p10[i], t0 = 8 * p01[i] + p00[i];
+                                    const float S = __builtin_fmaf((float)t1, 256.0f, (float)t0);
+                                    acc[c][i] = q4k_epi(acc[c][i], dx[k], f.d, S, f.dmin, s2[i]);
+                                } else {
+                                    const float S = __builtin_fmaf((float)(256 * p11[i] + p10[i]), 256.0f, (float)p00[i]);
+                                    acc[c][i] = __builtin_fmaf(dx[k], f.d * S, acc[c][i]);
+                                }
+                            }
+                            dx = nx;
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if constexpr (HALF) {
+                        // stage block 2 NB: a1 rows 0..15, a0 rows 16..31 of up to
+                        // 16 tokens; a lane's rows i and i + 8 are the two digits
+                        // of one token
+                        const uint8_t *ab = st + 2 * NB * XG_ABLK;
+                        v4i ah[XG_AHEAD];
+#pragma unroll
+                        for (int i = 0; i < XG_AHEAD; i++) ah[i] = read_a(2 * NB, i);
+                        v16i ph = (v16i)(0), pl = (v16i)(0);
+                        v16f s2 = (v16f)(0.0f);
+#pragma unroll
+                        for (int i = 0; i < 8; i++) {
+                            __builtin_amdgcn_sched_barrier(0);
+                            const v4i x = ah[i % XG_AHEAD];
+                            ph = __builtin_amdgcn_mfma_i32_32x32x32_i8(x, f.hi[i], ph, 0, 0, 0);
+                            pl = __builtin_amdgcn_mfma_i32_32x32x32_i8(x, f.lo[i], pl, 0, 0, 0);
+                            if (i + XG_AHEAD < 8) ah[i % XG_AHEAD] = read_a(2 * NB, i + XG_AHEAD);
+                            if constexpr (F::MIN)
+                                if (i == 6) {
+                                    const h8 sm = *reinterpret_cast<const h8 *>(ab + XG_ABS + r32 * 32 + 16 * h);
+                                    s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(sm, f.bm, s2, 0, 0, 0);
+                                }
+                        }
+                        const f4 dx[2] = {*reinterpret_cast<const f4 *>(ab + XG_AD + 64 + 16 * h),
+                                          *reinterpret_cast<const f4 *>(ab + XG_AD + 96 + 16 * h)};
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int i = 0; i < 8; i++) {
+                            float o = acc[NB][i];
+                            if constexpr (F::MIN) {
+                                const int t1 = 8 * ph[i] + pl[i], t0 = 8 * ph[i + 8] + pl[i + 8];
+                                const float S = __builtin_fmaf((float)t1, 256.0f, (float)t0);
+                                o = q4k_epi(o, dx[i >> 2][i & 3], f.d, S, f.dmin,
+                                            __builtin_fmaf(s2[i], 256.0f, s2[i + 8]));
+                            } else {
+                                const int t1 = 256 * ph[i] + pl[i] + ph[i + 8];
+                                const float S = __builtin_fmaf((float)t1, 256.0f, (float)pl[i + 8]);
+                                o = __builtin_fmaf(dx[i >> 2][i & 3], f.d * S, o);
+                            }
+                            acc[NB][i] = o;
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                } else {
+                    v4i a[XG_AHEAD];
+#pragma unroll
+                    for (int i = 0; i < XG_AHEAD; i++) a[i] = read_a(i >> 3, i & 7);
+#pragma unroll
+                    for (int c = 0; c < NB; c++) {
+                        const uint8_t *ab = st + c * XG_ABLK;
+                        const h8 as = *reinterpret_cast<const h8 *>(ab + XG_ABS + r32 * 32 + 16 * h);
+                        v16i sh = (v16i)(0), sl = (v16i)(0);
+                        v16f s2;
+#pragma unroll
+                        for (int i = 0; i < 8; i++) {
+                            __builtin_amdgcn_sched_barrier(0);
+                            const v4i ai = a[i % XG_AHEAD];
+                            sh = __builtin_amdgcn_mfma_i32_32x32x32_i8(ai, f.hi[i], sh, 0, 0, 0);
+                            sl = __builtin_amdgcn_mfma_i32_32x32x32_i8(ai, f.lo[i], sl, 0, 0, 0);
+                            const int n = 8 * c + i + XG_AHEAD;
+                            if (n < 8 * NB) a[i % XG_AHEAD] = read_a(n >> 3, n & 7);
+                            if (i == 6) s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(as, f.bm, (v16f)(0.0f), 0, 0, 0);
+                        }
+                        // lane: weight row r32, activation rows 8 j + 4 h + i
+                        f4 dx = *reinterpret_cast<const f4 *>(ab + XG_AD + 16 * h);
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            f4 nx = dx;
+                            __builtin_amdgcn_sched_barrier(0);
+                            if (j < 3) nx = *reinterpret_cast<const f4 *>(ab + XG_AD + 32 * (j + 1) + 16 * h);
+#pragma unroll
+                            for (int i = 0; i < 4; i++) {
+                                const int isum = 8 * sh[4 * j + i] + sl[4 * j + i];
+                                acc[c][4 * j + i] = q4k_epi(acc[c][4 * j + i], dx[i], f.d, (float)isum, f.dmin, s2[4 * j + i]);
+                            }
+                            dx = nx;
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                stg = stg == LEAD ? 0 : stg + 1;
             }
-#pragma unroll
-            for (int c = 0; c < XG_NC; c++)
-                if (c < I.nblk) xg_products(f, st + XG_WBYTES + c * ASTEP_BYTES, r16, g, acc[c]);
-            stg ^= 1;
+        };
+        typedef std::integral_constant<int, 0> zero;
+        typedef std::integral_constant<int, 1> one;
+        if constexpr (MERGE) {
+            switch (I.nblk >> 1) {
+            case 1: run(zero(), one()); break;
+            case 2: run(one(), zero()); break;
+            case 3: run(one(), one()); break;
+            default: run(std::integral_constant<int, 2>(), zero()); break;
+            }
+        } else {
+            switch ((I.nblk + 1) >> 1) {
+            case 1: run(one(), zero()); break;
+            case 2: run(std::integral_constant<int, 2>(), zero()); break;
+            case 3: run(std::integral_constant<int, 3>(), zero()); break;
+            default: run(std::integral_constant<int, 4>(), zero()); break;
+            }
         }
 
-        const int32_t *pids = s_pids[buf];
+        // Results.  Lane: weight row r32; activation rows (MERGE: tokens) 32 c +
+        // 8 j + 4 h + i, i < 4 (shared: the digits of token 16 c + 4 j + 2 h + i / 2).
+        // (the lane's row goes through an empty asm, so that the compiler does
+        // not hold every row's index in registers across the steps)
+        const int32_t *pids = s_pids[pb];
+        int hr = h, odd = (lane >> 4) & 1;
+        asm volatile("" : "+v"(hr), "+v"(odd));
         if (!DOWN) {
-            // h = silu(gate) * up, f32 (the two digits of a shared token summed)
+            // h = silu(gate) * up, f32.  Lanes 0..15 of each 32 hold gate row
+            // r16, lanes 16..31 up row r16: v_permlane16_swap of rows (a, b)
+            // leaves gate of a (lanes 0..15) and of b (16..31) in the first,
+            // up of both in the second
             const int col = I.rg * XG_GU_ROWS + 16 * wave + r16;
+            auto swap = [](float &a, float &b) {
+                const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a),
+                                                                __builtin_bit_cast(unsigned, b), false, false);
+                const unsigned r0 = r[0], r1 = r[1];
+                a = __builtin_bit_cast(float, r0);
+                b = __builtin_bit_cast(float, r1);
+            };
 #pragma unroll
-            for (int c = 0; c < XG_NC; c++) {
-                if (c >= I.nblk) continue;
-                if (!I.shared) {
+            for (int c = 0; c < NBMAX; c++) {
+                if ((MERGE ? 4 : 2) * c >= I.nblk) continue;
+                if (MERGE || !I.shared) {
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int q = EXPERT_CHUNK * c + 4 * g + i;
-                        if (q < I.nt) job.h[(size_t)pids[q] * FF + col] = silu(acc[c][0][i]) * acc[c][1][i];
+                    for (int i = 0; i < 16; i += 2) {
+                        float a = acc[c][i], b = acc[c][i + 1];
+                        swap(a, b);
+                        const int q = 32 * c + 8 * (i >> 2) + 4 * hr + (i & 3) + odd;
+                        if (q >= I.nt) continue;
+                        float *o = MERGE ? job.hs + (size_t)(I.t_first + q) * job.SF : job.h + (size_t)pids[q] * FF;
+                        o[col] = silu(a) * b;
                     }
                 } else {
 #pragma unroll
-                    for (int i = 0; i < 4; i += 2) {
-                        const int q = SHARED_CHUNK * c + 2 * g + (i >> 1);
-                        if (q < I.nt)
-                            job.hs[(size_t)(I.t_first + q) * job.SF + col] =
-                                silu(acc[c][0][i] + acc[c][0][i + 1]) * (acc[c][1][i] + acc[c][1][i + 1]);
+                    for (int i = 0; i < 16; i += 4) {
+                        float a = acc[c][i] + acc[c][i + 1], b = acc[c][i + 2] + acc[c][i + 3];
+                        swap(a, b);
+                        const int q = 16 * c + i + 2 * hr + odd;
+                        if (q < I.nt) job.hs[(size_t)(I.t_first + q) * job.SF + col] = silu(a) * b;
                     }
                 }
             }
         } else {
-            const int row0 = I.rg * XG_DN_ROWS + 32 * wave + r16;
+            const int row = I.rg * XG_DN_ROWS + 32 * wave + r32;
             float *out = I.shared ? job.ys + (size_t)slice * N * H : job.ye;
 #pragma unroll
-            for (int c = 0; c < XG_NC; c++) {
-                if (c >= I.nblk) continue;
-                if (!I.shared) {
+            for (int c = 0; c < NBMAX; c++) {
+                if ((MERGE ? 4 : 2) * c >= I.nblk) continue;
+                if (MERGE || !I.shared) {
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int q = EXPERT_CHUNK * c + 4 * g + i;
-                        if (q < I.nt) {
-                            float *op = out + (size_t)pids[q] * H + row0;
-                            op[0] = acc[c][0][i];
-                            op[16] = acc[c][1][i];
-                        }
+                    for (int i = 0; i < 16; i++) {
+                        const int q = 32 * c + 8 * (i >> 2) + 4 * hr + (i & 3);
+                        if (q < I.nt) out[(size_t)(MERGE ? I.t_first + q : pids[q]) * H + row] = acc[c][i];
                     }
                 } else {
 #pragma unroll
-                    for (int i = 0; i < 4; i += 2) {
-                        const int q = SHARED_CHUNK * c + 2 * g + (i >> 1);
-                        if (q < I.nt) {
-                            float *op = out + (size_t)(I.t_first + q) * H + row0;
-                            op[0] = acc[c][0][i] + acc[c][0][i + 1];
-                            op[16] = acc[c][1][i] + acc[c][1][i + 1];
-                        }
+                    for (int i = 0; i < 16; i += 2) {
+                        const int q = 16 * c + 4 * (i >> 2) + 2 * hr + ((i >> 1) & 1);
+                        if (q < I.nt) out[(size_t)(I.t_first + q) * H + row] = acc[c][i] + acc[c][i + 1];
                     }
                 }
             }
         }
         if (!NI.valid) break;
+        // (every wavefront has passed this item's first barrier: none reads
+        // the list of the item before it any more)
+        if (tid < XG_CHUNK) s_pids[pb2][tid] = npid;
         I = NI;
+        NI = NNI;
         slice = nslice;
-        k += G;
-        buf ^= 1;
-        NI = xg_decode(job, (k + G) / KS, rg_n, n_ec, nch);
-        nslice = (k + G) % KS;
+        round++;
+        nslice = k % KS;
+        pb = pb1;
     }
     // every wavefront leaves with no loads in flight
     EXPERT_WAIT_VM(0);
@@ -393,10 +734,18 @@ hipError_t launch_expert_gemm_q4k(int phase, const MoeJob &job, hipStream_t s)
     const hipError_t e = device_cu_count(&n_cu);
     if (e != hipSuccess) return e;
     const int grid = ((n_cu + 7) / 8) * 8;
-    if (phase == 0)
-        hipLaunchKernelGGL(k_gemm_q4k<false>, dim3(grid), dim3(XG_WAVES * 64), 0, s, job);
-    else
-        hipLaunchKernelGGL(k_gemm_q4k<true>, dim3(grid), dim3(XG_WAVES * 64), 0, s, job);
+    const dim3 gd(grid), bd(XG_WAVES * 64);
+    if (!routed) {
+        if (phase == 0)
+            hipLaunchKernelGGL((k_gemm_q<XgQ4K, false, true>), gd, bd, 0, s, job);
+        else
+            hipLaunchKernelGGL((k_gemm_q<XgQ4K, true, true>), gd, bd, 0, s, job);
+    } else {
+        if (phase == 0)
+            hipLaunchKernelGGL((k_gemm_q<XgQ4K, false, false>), gd, bd, 0, s, job);
+        else
+            hipLaunchKernelGGL((k_gemm_q<XgQ4K, true, false>), gd, bd, 0, s, job);
+    }
     return hipGetLastError();
 }
 

@@ -65,9 +65,12 @@ __device__ __forceinline__ int block_scan(int v, int *s_tmp, int *total)
 __device__ void dispatch_lists(int c, const RouteParams &rp, const RouteBufs &rb,
                                const WorkList &wl, int *s_tmp, int *s_off, bool publish)
 {
+    __shared__ int s_cls[8][RT_WAVES];
     const int E = rp.n_experts, tid = threadIdx.x;
     int total, nec, off, ecb;
-    const int nch = (c + wl.chunk - 1) / wl.chunk;
+    // by_size: the scan places the whole chunks; the remainders follow
+    const int rem = wl.by_size ? c % wl.chunk : 0;
+    const int nch = wl.by_size ? c / wl.chunk : (c + wl.chunk - 1) / wl.chunk;
     if (rp.n_tokens * rp.top_k < 32768 && E + rp.n_tokens * rp.top_k / wl.chunk + 1 < 32768) {
         // both prefixes in one scan (pair counts in the low 16 bits, chunk
         // counts in the high ones): every partial sum of either is below 2^15
@@ -89,6 +92,33 @@ __device__ void dispatch_lists(int c, const RouteParams &rp, const RouteBufs &rb
             wl.ec_expert[ecb + k] = tid;
             wl.ec_chunk[ecb + k] = k;
         }
+    }
+    if (wl.by_size) {
+        // remainders by class (eighths of a chunk, 1 .. 8), the largest first,
+        // then by expert: ranks from ballots and the wavefronts' class counts
+        const int lane = tid & 63, wave = tid >> 6, nw = (E + 63) / 64;
+        const int cls = tid < E && rem ? (8 * rem + wl.chunk - 1) / wl.chunk : 0;
+        int below = 0;
+#pragma unroll
+        for (int k = 1; k <= 8; k++) {
+            const uint64_t m = __ballot(cls == k);
+            if (cls == k)
+                below = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            if (lane == 0) s_cls[k - 1][wave] = __popcll(m);
+        }
+        __syncthreads();
+        int before = 0, all = 0;
+        for (int k = 1; k <= 8; k++)
+            for (int w = 0; w < nw; w++) {
+                const int n = s_cls[k - 1][w];
+                before += k > cls || (k == cls && w < wave) ? n : 0;
+                all += n;
+            }
+        if (publish && cls) {
+            wl.ec_expert[nec + before + below] = tid;
+            wl.ec_chunk[nec + before + below] = nch;
+        }
+        nec += all;
     }
     if (publish && tid == 0) {
         rb.offsets[E] = total;

@@ -1,0 +1,47 @@
+"""GPU parity of the grouped GEMM over units of tokens (projections past the
+few-token kernel: the LM head, the dense MLP): units of 64 tokens in two
+blocks of 32, the last a half block of 16, each partly filled, whole, or just
+begun.
+
+Bars (max|y - y_oracle| / max|y_oracle|): as the projections' other tests,
+exact weights times the activations as two int8 digits: 5e-4."""
+import numpy as np
+import pytest
+
+from conftest import max_rel_err
+
+pytestmark = pytest.mark.gpu
+
+TOL = 5e-4
+WTYPES = [12]
+
+
+@pytest.mark.parametrize("wtype", WTYPES)
+@pytest.mark.parametrize("N", [33, 48, 63, 64, 65, 97, 128])
+def test_head_units(ctx, O, wtype, N):
+    from dmoe import synth
+    H, V = 512, 1280            # two super-blocks: the shortest reduction; five row groups
+    print(f"case: LM head H={H} V={V} type={wtype} N={N}", flush=True)
+    w = synth.host_head(H, V, wtype, 20 + N, O.quantize_rows)
+    h = (synth.normal(21 + N, synth.S_X, N * H).reshape(N, H) * 2).astype(np.float32)
+    head = ctx.head_upload(w)
+    lg = ctx.head_forward(head, h, 1e-6, logits=True)[2]
+    err = max_rel_err(lg, O.head_forward(w, h, 1e-6)[2])
+    print(f"  max rel err {err:.3e}", flush=True)
+    assert err <= TOL
+    head.free()
+
+
+@pytest.mark.parametrize("wtype", WTYPES)
+@pytest.mark.parametrize("N", [33, 64, 90, 129])
+def test_dense_units(ctx, O, wtype, N):
+    from dmoe import synth
+    H, FF = 1024, 1536          # twelve row groups of h, a down reduction in slices
+    print(f"case: dense MLP H={H} n_ff={FF} type={wtype} N={N}", flush=True)
+    w = synth.host_dense(H, FF, wtype, 30 + N, O.quantize_rows)
+    x = synth.normal(31 + N, synth.S_X, N * H).reshape(N, H)
+    layer = ctx.dense_upload(w)
+    err = max_rel_err(ctx.forward(layer, x), O.dense_forward(w, x))
+    print(f"  max rel err {err:.3e}", flush=True)
+    assert err <= TOL
+    layer.free()
