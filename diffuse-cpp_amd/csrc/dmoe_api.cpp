@@ -1104,7 +1104,13 @@ bool dense_few(int path, int H, int FF, int N)
     return (path == DP_Q4K || path == DP_Q6K) && proj_ok(FF, H, N) && proj_ok(H, FF, N) && FF % 256 == 0;
 }
 
-int dense_chunk(int path, int N) { return path == DP_Q6K ? std::min(N, PROJ_MAX_TOKENS) : N; }
+int dense_gemm_slices(const KernelSwitches &sw, int path, int H, int FF, int N);
+
+// (Q6_K shapes that the GEMM does not take)
+int dense_chunk(const KernelSwitches &sw, int path, int H, int FF, int N)
+{
+    return path == DP_Q6K && !dense_gemm_slices(sw, path, H, FF, N) ? std::min(N, PROJ_MAX_TOKENS) : N;
+}
 
 // Slice-sum floats the few-token projection of R x K (M matrices) needs at
 // any token count 1 .. nmax (a smaller last chunk may split its reduction
@@ -1138,8 +1144,6 @@ size_t proj_partial_max(int R, int K, int M, int nmax, bool split_only)
     return best;
 }
 
-int dense_gemm_slices(const KernelSwitches &sw, int path, int H, int FF, int N);
-
 size_t plan_dense(const KernelSwitches &sw, const dmoe_layer *L, int N, bool host_io, uint8_t *base, DenseWs *w)
 {
     const int H = L->hp.n_embd, FF = L->hp.shared_ff;
@@ -1159,8 +1163,8 @@ size_t plan_dense(const KernelSwitches &sw, const dmoe_layer *L, int N, bool hos
     switch (path) {
     case DP_Q4K:
     case DP_Q6K: {
-        // Q6_K: workspace for one chunk of tokens, reused chunk after chunk
-        const int n = dense_chunk(path, N);
+        // Q6_K in chunks: workspace for one, reused chunk after chunk
+        const int n = dense_chunk(sw, path, H, FF, N);
         t.axs = take_act(take, n, H, true);
         t.ahs = take_act(take, n, FF, true);
         if (dense_few(path, H, FF, n)) {
@@ -1219,11 +1223,11 @@ int enqueue_dense(dmoe_ctx *ctx, const dmoe_layer *L, const DenseWs &w, const fl
         STAGE(ST_SH_DOWN, launch_down_shared(L->sd, w.hs, N, FF, H, y, s));
         return DMOE_OK;
     }
-    if (dense_few(path, H, FF, dense_chunk(path, N))) {
+    if (dense_few(path, H, FF, dense_chunk(ctx->sw, path, H, FF, N))) {
         // gate and up: one launch over both matrices, h from their slices;
-        // tokens t0 .. t0 + n - 1 at a time (every token at once for Q4_K)
+        // tokens t0 .. t0 + n - 1 at a time (every token at once, or Q6_K chunks)
         const bool q6 = path == DP_Q6K;
-        const int nc = dense_chunk(path, N);
+        const int nc = dense_chunk(ctx->sw, path, H, FF, N);
         for (int t0 = 0; t0 < N; t0 += nc) {
             const int n = std::min(nc, N - t0);
             ProjJob gu{};
@@ -1258,7 +1262,7 @@ int enqueue_dense(dmoe_ctx *ctx, const dmoe_layer *L, const DenseWs &w, const fl
         return DMOE_OK;
     }
     if (const int ks = dense_gemm_slices(ctx->sw, path, H, FF, N)) {
-        // many tokens of Q4_K: the grouped GEMM's gate/up and down launches
+        // many tokens of Q4_K or Q6_K: the grouped GEMM's gate/up and down launches
         // over shared units (no routed work list), h converted between them,
         // the down reduction in slices added in order
         WorkList wl{};
@@ -1370,12 +1374,8 @@ struct ProjWs {
     float *part;                         // slice sums of the few-token Q4_K projection
 };
 
-// Tokens per launch of a projection: Q6_K runs only the few-token kernel,
-// in chunks of up to PROJ_MAX_TOKENS tokens.
-int proj_chunk(int path, int N) { return path == DP_Q6K ? std::min(N, PROJ_MAX_TOKENS) : N; }
-
-// Q4_K projections of PROJ_GEMM_MIN_TOKENS or more tokens run on the grouped
-// GEMM's down launch (k_expert_gemm.hip) with shared units only: 64 tokens
+// Q4_K and Q6_K projections of PROJ_GEMM_MIN_TOKENS or more tokens run on the
+// grouped GEMM's down launch (k_expert_gemm.hip) with shared units only: 64 tokens
 // (128 digit rows) per unit, 256 output rows per item, the reduction split
 // into slices of 2 or more super-blocks, as many as minimise the static
 // schedule's rounds x steps plus the slices' own traffic.  Returns the slice
@@ -1384,7 +1384,7 @@ constexpr int PROJ_GEMM_MIN_TOKENS = 33;
 
 int proj_gemm_slices(const KernelSwitches &sw, int path, int rows, int K, int N)
 {
-    if (path != DP_Q4K || sw.proj_gemm == 0 || (sw.proj_gemm < 0 && N < PROJ_GEMM_MIN_TOKENS) ||
+    if ((path != DP_Q4K && path != DP_Q6K) || sw.proj_gemm == 0 || (sw.proj_gemm < 0 && N < PROJ_GEMM_MIN_TOKENS) ||
         !expert_gemm_q4k_ok(rows, K, K, true) || 2L * N * K >= (1L << 31))
         return 0;
     int n_cu = 0;
@@ -1409,6 +1409,13 @@ int proj_gemm_slices(const KernelSwitches &sw, int path, int rows, int K, int N)
     return best;
 }
 
+// Tokens per launch of a projection: every token, or, for Q6_K shapes that the
+// GEMM does not take, chunks of up to PROJ_MAX_TOKENS of the few-token kernel.
+int proj_chunk(const KernelSwitches &sw, int path, int rows, int K, int N)
+{
+    return path == DP_Q6K && !proj_gemm_slices(sw, path, rows, K, N) ? std::min(N, PROJ_MAX_TOKENS) : N;
+}
+
 // The dense MLP past the few-token kernels on the same GEMM (gate/up, then
 // down in proj_gemm_slices slices): 0 where it does not take the shape.
 int dense_gemm_slices(const KernelSwitches &sw, int path, int H, int FF, int N)
@@ -1425,7 +1432,7 @@ ProjWs plan_proj(const KernelSwitches &sw, int path, int N, int K, int rows, Tak
     switch (path) {
     case DP_Q4K:
     case DP_Q6K: {
-        const int n = proj_chunk(path, N);
+        const int n = proj_chunk(sw, path, rows, K, N);
         p.act = take_act(take, n, K, true);
         if (proj_ok(rows, K, n)) {
             if (const size_t pf = proj_partial_max(rows, K, 1, n, true)) p.part = (float *)take(pf * 4);
@@ -1535,9 +1542,9 @@ int enqueue_proj(dmoe_ctx *ctx, bool prof, int st_conv, int st_prod, const WTens
         STAGE(st_prod, launch_down_shared(W, x, N, K, rows, y, s));
         return DMOE_OK;
     }
-    if (proj_few(path, rows, K, proj_chunk(path, N))) {
+    if (proj_few(path, rows, K, proj_chunk(ctx->sw, path, rows, K, N))) {
         // every token at once, or (Q6_K) chunks of up to PROJ_MAX_TOKENS
-        const int nc = proj_chunk(path, N);
+        const int nc = proj_chunk(ctx->sw, path, rows, K, N);
         for (int t0 = 0; t0 < N; t0 += nc) {
             const int n = std::min(nc, N - t0);
             PrepJob pj{x + (size_t)t0 * K, n, K, ACT_SPLIT, p.act};
@@ -1548,7 +1555,7 @@ int enqueue_proj(dmoe_ctx *ctx, bool prof, int st_conv, int st_prod, const WTens
         return DMOE_OK;
     }
     if (const int ks = proj_gemm_slices(ctx->sw, path, rows, K, N)) {
-        // many tokens of Q4_K: the grouped GEMM's down launch over shared
+        // many tokens of Q4_K or Q6_K: the grouped GEMM's down launch over shared
         // units, its reduction slices added in order
         PrepJob pj{x, N, K, ACT_SPLIT, p.act};
         STAGE(st_conv, launch_prep(&pj, 1, s));

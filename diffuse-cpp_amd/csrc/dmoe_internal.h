@@ -132,7 +132,7 @@ struct MoeJob {
 //   DMOE_GATEUP_LDS = 1               the LDS-ring gate/up kernel instead of the register ring
 //   DMOE_EXPERT_TILE = 0 / 1          the tile kernels (k_expert_tile.hip) off / on for every N
 //   DMOE_EXPERT_GEMM = 0 / 1          the Q4_K grouped GEMM (k_expert_gemm.hip) off / on for every N
-//   DMOE_PROJ_GEMM = 0 / 1            Q4_K projections (attention, LM head) past the few-token
+//   DMOE_PROJ_GEMM = 0 / 1            Q4_K and Q6_K projections (attention, LM head, dense MLP) past the few-token
 //                                     kernel on that GEMM off / on for every N
 struct KernelSwitches {
     int q4k_column_blocks = 0;

@@ -13,7 +13,7 @@ from conftest import max_rel_err
 pytestmark = pytest.mark.gpu
 
 TOL = 5e-4
-WTYPES = [12]
+WTYPES = [12, 14]
 
 
 @pytest.mark.parametrize("wtype", WTYPES)
