@@ -1382,9 +1382,22 @@ struct ProjWs {
 // count, 0 where the GEMM does not take the shape.
 constexpr int PROJ_GEMM_MIN_TOKENS = 33;
 
+// Q6_K matrices of an LM head's rows take the GEMM (in units of 32 tokens)
+// from 17 tokens on: at 157,184 x 4,096 rows 16 / 17 / 24 / 32 tokens 145 / 167
+// / 172 / 177 us against 140 / 174 / 177 / 217 on the few-token kernel, whose
+// work per weight grows by the eight tokens.  A few thousand rows fill too few
+// of the GEMM's 256-row items.
+constexpr int PROJ_GEMM_MIN_TOKENS_Q6K_HEAD = 17;
+
+int proj_gemm_min_tokens(int path, int rows)
+{
+    return path == DP_Q6K && rows > PROJ_ROWS_MAX ? PROJ_GEMM_MIN_TOKENS_Q6K_HEAD : PROJ_GEMM_MIN_TOKENS;
+}
+
 int proj_gemm_slices(const KernelSwitches &sw, int path, int rows, int K, int N)
 {
-    if ((path != DP_Q4K && path != DP_Q6K) || sw.proj_gemm == 0 || (sw.proj_gemm < 0 && N < PROJ_GEMM_MIN_TOKENS) ||
+    if ((path != DP_Q4K && path != DP_Q6K) || sw.proj_gemm == 0 ||
+        (sw.proj_gemm < 0 && N < proj_gemm_min_tokens(path, rows)) ||
         !expert_gemm_q4k_ok(rows, K, K, true) || 2L * N * K >= (1L << 31))
         return 0;
     int n_cu = 0;
@@ -1424,6 +1437,8 @@ int dense_gemm_slices(const KernelSwitches &sw, int path, int H, int FF, int N)
     return proj_gemm_slices(sw, path, H, FF, N);
 }
 
+bool proj_few(const KernelSwitches &sw, int path, int rows, int K, int N);
+
 template <class Take>
 ProjWs plan_proj(const KernelSwitches &sw, int path, int N, int K, int rows, Take &&take)
 {
@@ -1434,7 +1449,7 @@ ProjWs plan_proj(const KernelSwitches &sw, int path, int N, int K, int rows, Tak
     case DP_Q6K: {
         const int n = proj_chunk(sw, path, rows, K, N);
         p.act = take_act(take, n, K, true);
-        if (proj_ok(rows, K, n)) {
+        if (proj_few(sw, path, rows, K, n)) {
             if (const size_t pf = proj_partial_max(rows, K, 1, n, true)) p.part = (float *)take(pf * 4);
         } else if (const int ks = proj_gemm_slices(sw, path, rows, K, N); ks > 1) {
             p.part = (float *)take((size_t)ks * N * rows * 4);
@@ -1450,9 +1465,10 @@ ProjWs plan_proj(const KernelSwitches &sw, int path, int N, int K, int rows, Tak
 
 // Few tokens of Q4_K or Q6_K weights: k_proj.hip on x already converted to
 // p.act.
-bool proj_few(int path, int rows, int K, int N)
+bool proj_few(const KernelSwitches &sw, int path, int rows, int K, int N)
 {
-    return (path == DP_Q4K || path == DP_Q6K) && proj_ok(rows, K, N);
+    if ((path != DP_Q4K && path != DP_Q6K) || !proj_ok(rows, K, N)) return false;
+    return N < proj_gemm_min_tokens(path, rows) || !proj_gemm_slices(sw, path, rows, K, N);
 }
 
 // y [N][rows] = W x from p.act: 128 T-row tiles x reduction slices over every
@@ -1521,7 +1537,7 @@ int enqueue_proj_gemm(dmoe_ctx *ctx, bool prof, int st_prod, const WTensor &W, i
 bool proj_takes_digits(const KernelSwitches &sw, int path, int rows, int K, int N, int *gemm_ks)
 {
     *gemm_ks = 0;
-    if (proj_few(path, rows, K, N)) return true;
+    if (proj_few(sw, path, rows, K, N)) return true;
     *gemm_ks = proj_gemm_slices(sw, path, rows, K, N);
     return *gemm_ks > 0;
 }
@@ -1542,7 +1558,7 @@ int enqueue_proj(dmoe_ctx *ctx, bool prof, int st_conv, int st_prod, const WTens
         STAGE(st_prod, launch_down_shared(W, x, N, K, rows, y, s));
         return DMOE_OK;
     }
-    if (proj_few(path, rows, K, proj_chunk(ctx->sw, path, rows, K, N))) {
+    if (proj_few(ctx->sw, path, rows, K, proj_chunk(ctx->sw, path, rows, K, N))) {
         // every token at once, or (Q6_K) chunks of up to PROJ_MAX_TOKENS
         const int nc = proj_chunk(ctx->sw, path, rows, K, N);
         for (int t0 = 0; t0 < N; t0 += nc) {

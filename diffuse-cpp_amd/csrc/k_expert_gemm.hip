@@ -87,7 +87,6 @@ constexpr int XG_DN_ROWS = XG_WAVES * 32;                    // n_embd rows of a
 constexpr int XG_ABS = 8 * 1024 + 3 * 64;                    // sums of 16: [32][16] f16
 constexpr int XG_AD = XG_ABS + 1024;                         // scales: [32] f32
 constexpr int XG_ABLK = XG_AD + 128;                         // one block (9,344)
-constexpr int XG_ASTAGE = (XG_NC / 2) * XG_ABLK;
 constexpr int XG_AHEAD = 4;                                  // operand reads ahead of their MFMAs (divides 8)
 static_assert(XG_ABLK % 16 == 0, "16-byte pieces");
 
@@ -98,7 +97,7 @@ struct XgItem {
     bool shared, valid;
 };
 
-template <bool MERGE>
+template <bool MERGE, int SCHUNK = XG_SCHUNK>
 __device__ __forceinline__ XgItem xg_decode(const MoeJob &job, int k, int rg_n, int n_ec, int nch)
 {
     XgItem I{};
@@ -115,8 +114,8 @@ __device__ __forceinline__ XgItem xg_decode(const MoeJob &job, int k, int rg_n, 
         I.nblk = (I.nt + EXPERT_CHUNK - 1) / EXPERT_CHUNK;
     } else {
         I.e = 0;
-        I.t_first = unit * XG_SCHUNK;
-        I.nt = min(XG_SCHUNK, job.n_tokens - I.t_first);
+        I.t_first = unit * SCHUNK;
+        I.nt = min(SCHUNK, job.n_tokens - I.t_first);
         // MERGE: 32-token blocks (four 16-row blocks), the last one a half
         // block (two) when it holds up to 16 tokens
         I.nblk = MERGE ? 2 * ((I.nt + 15) / 16) : (I.nt + SHARED_CHUNK - 1) / SHARED_CHUNK;
@@ -334,12 +333,24 @@ struct XgQ6K {
     }
 };
 
-template <class F, bool DOWN, bool MERGE>
+// FEW: units of 32 tokens (MERGE), whose smaller activation stages leave room
+// for two stages of weights: with few tokens a step lasts no longer than a CU's
+// weights take to arrive, and one stage, refilled only while a step's products
+// run, stalls it (LM head of Q6_K, 157,184 x 4,096, at 32 tokens: 190 us with
+// one stage, 177 with two; the fold is the larger part of what is left).
+// (Measured and not kept: the same for the routed Q4_K experts, units of 64
+// pairs, from 256 tokens: 292 us against 269 on the tile kernels.)
+template <class F, bool DOWN, bool MERGE, bool FEW = false>
 __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
 {
-    constexpr int NBMAX = MERGE ? XG_NC / 4 : XG_NC / 2;   // 32-row (MERGE: 32-token) blocks of a unit
+    static_assert(!FEW || (MERGE && F::ASTAGES == 2), "weight stages beside two activation stages");
+    constexpr int NC = FEW ? XG_NC / 2 : XG_NC, SCHUNK = FEW ? XG_SCHUNK / 2 : XG_SCHUNK;
+    constexpr int NBMAX = MERGE ? NC / 4 : NC / 2;         // 32-row (MERGE: 32-token) blocks of a unit
+    constexpr int XG_ASTAGE = (NC / 2) * XG_ABLK;          // bytes of an activation stage
+    constexpr int WST = FEW ? 2 : 1;                       // weight stages
+    constexpr int WLOADS = 2 * ((F::TILE + 1023) / 1024);  // loads of a weight stage
     __shared__ __align__(16) uint8_t SA[F::ASTAGES][XG_ASTAGE];
-    __shared__ __align__(16) uint8_t SW[XG_WAVES][2 * F::TLDS];
+    __shared__ __align__(16) uint8_t SW[XG_WAVES][WST][2 * F::TLDS];
     // pair ids of the routed items i, i + 1 (its activations load during
     // item i) and i + 2 (read from perm during item i, written at its end)
     __shared__ int32_t s_pids[3][XG_CHUNK];
@@ -349,7 +360,7 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
     const int r16 = lane & 15, r32 = lane & 31, h = lane >> 5;
     const int H = job.H, FF = job.FF, N = job.n_tokens, K = job.top_k;
     const int n_ec = job.wl.n_ec ? ldc(job.wl.n_ec, 0) : 0;   // none: shared units only
-    const int nch = job.has_shared ? (N + XG_SCHUNK - 1) / XG_SCHUNK : 0;
+    const int nch = job.has_shared ? (N + SCHUNK - 1) / SCHUNK : 0;
     const int rg_n = DOWN ? H / XG_DN_ROWS : FF / XG_GU_ROWS;
     const int Kin = DOWN ? FF : H;
     // down launches of a projection split the reduction into KS slices of
@@ -359,11 +370,11 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
     const int G = gridDim.x;
 
     int k = schedule_item(blockIdx.x, G, 0), round = 0;
-    XgItem I = xg_decode<MERGE>(job, k / KS, rg_n, n_ec, nch);
+    XgItem I = xg_decode<MERGE, SCHUNK>(job, k / KS, rg_n, n_ec, nch);
     if (!I.valid) return;
     int slice = k % KS;
     k = schedule_item(blockIdx.x, G, 1);
-    XgItem NI = xg_decode<MERGE>(job, k / KS, rg_n, n_ec, nch);
+    XgItem NI = xg_decode<MERGE, SCHUNK>(job, k / KS, rg_n, n_ec, nch);
     int nslice = k % KS;
     if (tid < XG_CHUNK && !I.shared) s_pids[0][tid] = job.perm[I.t_first + min(tid, I.nt - 1)];
     if (tid < XG_CHUNK && NI.valid && !NI.shared) s_pids[1][tid] = job.perm[NI.t_first + min(tid, NI.nt - 1)];
@@ -373,7 +384,7 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
     // products, the activations two.  Wave-uniform bases; wavefront w loads
     // 16-row block w of the items that have it, by this lane's byte offsets
     // (32-bit: the host keeps every activation array below 2 GiB).
-    const uint32_t sw = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)&SW[wave][0];
+    const uint32_t sw0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)&SW[wave][0][0];
     const uint32_t sa = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)&SA[0][0];
     const uint8_t *wb0 = nullptr, *wb1 = nullptr;
     const uint8_t *aqb = nullptr, *absb = nullptr, *adb = nullptr;
@@ -413,10 +424,10 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
         abso = ((uint32_t)xg_arow<DOWN, MERGE>(C, pids, N, K, wave, (ln >> 1) & 15) * (uint32_t)(Kin / 16) + (ln & 1) * 8) * 2;
         ado = (uint32_t)xg_arow<DOWN, MERGE>(C, pids, N, K, wave, ln & 15) * (uint32_t)(Kin / 256) * 4;
     };
-    // the weight cursor's super-block to the wavefront's buffer; on to the next
-    auto issue_w = [&]() {
+    // the weight cursor's super-block to the wavefront's stage ws; on to the next
+    auto issue_w = [&](int ws) {
         constexpr int FULL = F::TILE / 1024, REST = (F::TILE % 1024) / 16;
-        const uint32_t vo = (uint32_t)lane * 16;
+        const uint32_t vo = (uint32_t)lane * 16, sw = sw0 + ws * (2 * F::TLDS);
 #pragma unroll
         for (int i = 0; i < FULL; i++) {
             xg_lds16(wb0, vo + 1024 * i, sw + 1024 * i);
@@ -451,13 +462,16 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
 #pragma unroll
     for (int c = 0; c < 4; c++)
         ao[c] = 1024 * (r32 >> 2) + 64 * (r32 >> 3) + 256 * (r32 & 3) + 64 * h + 16 * (c ^ (r32 & 3));
-    const uint8_t *wrd = &SW[wave][((lane >> 4) & 1) * F::TLDS];
+    const uint8_t *wrd = &SW[wave][0][((lane >> 4) & 1) * F::TLDS];
 
     weights_of(I, slice);
     acts_of(I, slice, s_pids[0]);
-    issue_w();
+    issue_w(0);
     issue_a(0);
     if (F::ASTAGES == 3) issue_a(1);                  // steps >= 2
+    if (FEW) issue_w(1);
+    int wst = 0;                                      // the weight stage the step reads
+    bool w_ahead = FEW;                               // weight loads issued after this step's activations
     int stg = 0;                                      // the stage the products read
     bool ahead = act_on;                              // activation loads issued after this step's weights
     int pb = 0;                                       // pair list of item I (of 3)
@@ -465,7 +479,7 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
     for (;;) {
         const int pb1 = pb == 2 ? 0 : pb + 1, pb2 = pb1 == 2 ? 0 : pb1 + 1;
         k = schedule_item(blockIdx.x, G, round + 2);
-        const XgItem NNI = xg_decode<MERGE>(job, k / KS, rg_n, n_ec, nch);
+        const XgItem NNI = xg_decode<MERGE, SCHUNK>(job, k / KS, rg_n, n_ec, nch);
         int npid = 0;
         if (tid < XG_CHUNK && NNI.valid && !NNI.shared) npid = job.perm[NNI.t_first + min(tid, NNI.nt - 1)];
 
@@ -482,34 +496,38 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
                 // this step's weights (this wavefront's) and activations
                 // (every wavefront's) have landed, the stage two steps on has
                 // been read by all
-                if (F::ASTAGES == 3 && ahead)
+                if (FEW && w_ahead)
+                    EXPERT_WAIT_VM(WLOADS);
+                else if (F::ASTAGES == 3 && ahead)
                     EXPERT_WAIT_VM(F::ALOADS);
                 else
                     EXPERT_WAIT_VM(0);
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
                 typename F::Raw t;
-                F::read(t, wrd, r16, h);
-                F::pin(t);                            // the buffer may be refilled
+                F::read(t, wrd + wst * (2 * F::TLDS), r16, h);
+                F::pin(t);                            // the stage may be refilled
                 // the stage the activations of step s + LEAD go to
                 constexpr int LEAD = F::ASTAGES - 1;
                 const int st2 = stg == 0 ? LEAD : stg - 1;
-                if (s + 1 < steps) {
-                    issue_w();
-                } else if (NI.valid) {
-                    weights_of(NI, nslice);
-                    issue_w();
-                }
-                if (s + LEAD < steps) {
-                    issue_a(st2);
-                    ahead = act_on;
-                } else if (NI.valid) {
+                auto next_w = [&]() {
+                    w_ahead = s + WST < steps || NI.valid;
+                    if (!w_ahead) return;
+                    if (s + WST == steps) weights_of(NI, nslice);
+                    issue_w(wst);
+                };
+                auto next_a = [&]() {
+                    ahead = false;
+                    if (s + LEAD >= steps && !NI.valid) return;
                     if (s + LEAD == steps) acts_of(NI, nslice, s_pids[pb1]);
                     issue_a(st2);
                     ahead = act_on;
-                } else {
-                    ahead = false;
-                }
+                };
+                // (the loads a wait leaves in flight are the last issued)
+                if (FEW) next_a();
+                next_w();
+                if (!FEW) next_a();
+                if (FEW) wst ^= 1;
                 typename F::Ops f;
                 F::fold(t, h, f);
                 // The blocks' products.  The operand reads run XG_AHEAD ahead
@@ -810,7 +828,9 @@ hipError_t launch_expert_gemm_q4k(int phase, const MoeJob &job, hipStream_t s)
     if (e != hipSuccess) return e;
     const int grid = ((n_cu + 7) / 8) * 8;
     const dim3 gd(grid), bd(XG_WAVES * 64);
-    if (ws.type == DMOE_TYPE_Q6_K && !routed) {
+    if (ws.type == DMOE_TYPE_Q6_K && !routed && phase == 1 && N <= XG_SCHUNK / 2) {
+        hipLaunchKernelGGL((k_gemm_q<XgQ6K, true, true, true>), gd, bd, 0, s, job);
+    } else if (ws.type == DMOE_TYPE_Q6_K && !routed) {
         if (phase == 0)
             hipLaunchKernelGGL((k_gemm_q<XgQ6K, false, true>), gd, bd, 0, s, job);
         else

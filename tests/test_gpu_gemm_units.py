@@ -45,3 +45,22 @@ def test_dense_units(ctx, O, wtype, N):
     print(f"  max rel err {err:.3e}", flush=True)
     assert err <= TOL
     layer.free()
+
+
+@pytest.mark.parametrize("H", [512, 1024])
+@pytest.mark.parametrize("N", [16, 17, 31, 32])
+def test_head_q6k_few_tokens(ctx, O, H, N):
+    """Q6_K heads of more than 32,768 rows: the GEMM's units of 32 tokens from
+    17 tokens on (one half block more than a whole one, whole blocks), the
+    few-token kernel below."""
+    from dmoe import synth
+    V = 33024                   # 129 row groups
+    print(f"case: LM head H={H} V={V} Q6_K N={N}", flush=True)
+    w = synth.host_head(H, V, 14, 40 + N, O.quantize_rows)
+    h = (synth.normal(41 + N, synth.S_X, N * H).reshape(N, H) * 2).astype(np.float32)
+    head = ctx.head_upload(w)
+    lg = ctx.head_forward(head, h, 1e-6, logits=True)[2]
+    err = max_rel_err(lg, O.head_forward(w, h, 1e-6)[2])
+    print(f"  max rel err {err:.3e}", flush=True)
+    assert err <= TOL
+    head.free()
