@@ -1374,7 +1374,7 @@ struct ProjWs {
     float *part;                         // slice sums of the few-token Q4_K projection
 };
 
-// Q4_K and Q6_K projections of PROJ_GEMM_MIN_TOKENS or more tokens run on the
+// Q4_K, Q6_K and Q8_0 projections of proj_gemm_min_tokens or more tokens run on the
 // grouped GEMM's down launch (k_expert_gemm.hip) with shared units only: 64 tokens
 // (128 digit rows) per unit, 256 output rows per item, the reduction split
 // into slices of 2 or more super-blocks, as many as minimise the static
@@ -1389,14 +1389,22 @@ constexpr int PROJ_GEMM_MIN_TOKENS = 33;
 // of the GEMM's 256-row items.
 constexpr int PROJ_GEMM_MIN_TOKENS_Q6K_HEAD = 17;
 
+// Q8_0 projections have no few-token kernel of their own: against the expert
+// kernel's items of 8 tokens the GEMM takes the attention half of 1 / 8 / 20
+// tokens from 95 / 98 / 99 us to 46 / 49 / 53, and an LM head of 16 / 32 tokens
+// from 233 / 468 us to 160 / 194; one item of the expert kernel covers a head
+// of up to 8 tokens (128 / 133 us at 1 / 8 tokens against 137 / 148).
+constexpr int PROJ_GEMM_MIN_TOKENS_Q80 = 1, PROJ_GEMM_MIN_TOKENS_Q80_HEAD = 9;
+
 int proj_gemm_min_tokens(int path, int rows)
 {
+    if (path == DP_Q80) return rows > PROJ_ROWS_MAX ? PROJ_GEMM_MIN_TOKENS_Q80_HEAD : PROJ_GEMM_MIN_TOKENS_Q80;
     return path == DP_Q6K && rows > PROJ_ROWS_MAX ? PROJ_GEMM_MIN_TOKENS_Q6K_HEAD : PROJ_GEMM_MIN_TOKENS;
 }
 
 int proj_gemm_slices(const KernelSwitches &sw, int path, int rows, int K, int N)
 {
-    if ((path != DP_Q4K && path != DP_Q6K) || sw.proj_gemm == 0 ||
+    if ((path != DP_Q4K && path != DP_Q6K && path != DP_Q80) || sw.proj_gemm == 0 ||
         (sw.proj_gemm < 0 && N < proj_gemm_min_tokens(path, rows)) ||
         !expert_gemm_q4k_ok(rows, K, K, true) || 2L * N * K >= (1L << 31))
         return 0;
@@ -1433,7 +1441,7 @@ int proj_chunk(const KernelSwitches &sw, int path, int rows, int K, int N)
 // down in proj_gemm_slices slices): 0 where it does not take the shape.
 int dense_gemm_slices(const KernelSwitches &sw, int path, int H, int FF, int N)
 {
-    if (2L * N * H >= (1L << 31)) return 0;
+    if (path == DP_Q80 || 2L * N * H >= (1L << 31)) return 0;
     return proj_gemm_slices(sw, path, H, FF, N);
 }
 
@@ -1456,7 +1464,10 @@ ProjWs plan_proj(const KernelSwitches &sw, int path, int N, int K, int rows, Tak
         }
         break;
     }
-    case DP_Q80: p.act = take_act(take, N, K, true, true); break;
+    case DP_Q80:
+        p.act = take_act(take, N, K, true, true);
+        if (const int ks = proj_gemm_slices(sw, path, rows, K, N); ks > 1) p.part = (float *)take((size_t)ks * N * rows * 4);
+        break;
     case DP_F16: p.x16 = (uint16_t *)take((size_t)2 * N * K * 2); break;
     default: break;
     }
@@ -1573,7 +1584,7 @@ int enqueue_proj(dmoe_ctx *ctx, bool prof, int st_conv, int st_prod, const WTens
     if (const int ks = proj_gemm_slices(ctx->sw, path, rows, K, N)) {
         // many tokens of Q4_K or Q6_K: the grouped GEMM's down launch over shared
         // units, its reduction slices added in order
-        PrepJob pj{x, N, K, ACT_SPLIT, p.act};
+        PrepJob pj{x, N, K, path == DP_Q80 ? ACT_SPLIT32 : ACT_SPLIT, p.act};
         STAGE(st_conv, launch_prep(&pj, 1, s));
         return enqueue_proj_gemm(ctx, prof, st_prod, W, rows, K, N, ks, p, y, nullptr, nullptr, s);
     }
@@ -1842,7 +1853,7 @@ int enqueue_attn(dmoe_ctx *ctx, const dmoe_layer *L, const AttnWs &w, const floa
     // :172 output projection; :175-178 residual, then the post-attention
     // layernorm (the MoE input)
     if (fo) {
-        PrepJob pj{w.att, N, QD, ACT_SPLIT, w.po.act};
+        PrepJob pj{w.att, N, QD, w.po.act.bs ? ACT_SPLIT : ACT_SPLIT32, w.po.act};
         STAGE(ST_ACTQ_H, launch_prep(&pj, 1, s));
         const float *o = w.proj;
         int oks = 1;

@@ -132,8 +132,8 @@ struct MoeJob {
 //   DMOE_GATEUP_LDS = 1               the LDS-ring gate/up kernel instead of the register ring
 //   DMOE_EXPERT_TILE = 0 / 1          the tile kernels (k_expert_tile.hip) off / on for every N
 //   DMOE_EXPERT_GEMM = 0 / 1          the Q4_K grouped GEMM (k_expert_gemm.hip) off / on for every N
-//   DMOE_PROJ_GEMM = 0 / 1            Q4_K and Q6_K projections (attention, LM head, dense MLP) past the few-token
-//                                     kernel on that GEMM off / on for every N
+//   DMOE_PROJ_GEMM = 0 / 1            Q4_K, Q6_K and Q8_0 projections (attention, LM head; Q4_K and Q6_K dense MLP)
+//                                     past the few-token kernels on that GEMM off / on for every N
 struct KernelSwitches {
     int q4k_column_blocks = 0;
     int expert_tile = -1;                // -1: by tokens per expert
@@ -191,7 +191,8 @@ hipError_t launch_tile_f16(const uint8_t *src, size_t nb1, size_t nb2, int rows,
 // x = rms_norm(h, eps) * gain (gain may be null).
 // rows of h_in (+ the sum of y's ks slices, kstride floats apart, written to
 // h_out when given) -> rms_norm * gain to x (f32, when given) and / or act
-// (two int8 digit rows per row, ACT_SPLIT, when act.q is given); H <= 8192
+// (two int8 digit rows per row, ACT_SPLIT, or ACT_SPLIT32 where act has no
+// sums, when act.q is given); H <= 8192
 struct NormArgs {
     const float *h_in;
     float *h_out;

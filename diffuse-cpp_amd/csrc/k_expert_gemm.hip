@@ -1,5 +1,5 @@
-// k_expert_gemm.hip — Q4_K and, in projections, Q6_K products as a grouped
-// int8-MFMA GEMM when many rows share each weight (prompt prefill and the sampler's large windows,
+// k_expert_gemm.hip — Q4_K and, in projections, Q6_K and Q8_0 products as a
+// grouped int8-MFMA GEMM when many rows share each weight (prompt prefill and the sampler's large windows,
 // N = 32 (blk + 1) of a thousand tokens and more):
 // src/diffuse-moe-graph.cpp:264-269 (ggml's mul_mat_id over Q4_K weights
 // with Q8_K activations), the shared expert of :280-286 (F32 activations
@@ -59,6 +59,7 @@
 // down products' int8 layout; the down products go to ye [pair][n_embd] /
 // ys [token][n_embd] for the combine launch, as with the tile kernels.
 #include "dmoe_q4k.h"
+#include "dmoe_q80.h"
 
 #include <type_traits>
 
@@ -173,15 +174,15 @@ __device__ __forceinline__ void xg_lds4(const void *base, uint32_t voff, uint32_
 //   TILE, TLDS, WLOADS   bytes of a 16-row tile's super-block in HBM, its
 //                        stride in LDS
 //   ASTAGES, ALOADS      activation stages; loads of a 16-row block
-//   MIN, BASE            a min term on the sums of 16; the two weight digits'
-//                        ratio
+//   MIN                  a min term on the sums of 16
+//   PER32                scales per 32 values (the products are XgQ80's)
 //   Raw, read, pin       the lane's bytes of a super-block, from LDS; in
 //                        registers from there on
 //   Ops, fold            the int8 operands: hi and lo digits of scale x quant,
 //                        chunk c of lane group 2 gp + h at [4 gp + c]
 struct XgQ4K {
     static constexpr int TILE = TILE_BYTES, TLDS = TILE_BYTES, ASTAGES = 3, ALOADS = 6;
-    static constexpr bool MIN = true;
+    static constexpr bool MIN = true, PER32 = false;
     struct Raw {
         uint4 h, q[4];
     };
@@ -269,7 +270,7 @@ struct XgQ4K {
 // us, of 40 tokens 120 -> 109.
 struct XgQ6K {
     static constexpr int TILE = 16 * Q6K_BYTES, TLDS = 14 * 256, ASTAGES = 2, ALOADS = 5;
-    static constexpr bool MIN = false;
+    static constexpr bool MIN = false, PER32 = false;
     struct Raw {
         uint4 q[6], sc;                  // L[0..3], L[4..7], H[0..3] of both lane groups; scales
         uint32_t d;
@@ -329,6 +330,55 @@ struct XgQ6K {
                     f.lo[4 * gp + c][i] = (int)(__builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u);
                 }
             }
+        }
+    }
+};
+
+// Q8_0 (tiled by launch_tile_q80, ACT_SPLIT32 activations), projections only:
+// the quants are the int8 operands as they lie, and a v_mfma_i32_32x32x32_i8 is
+// one 32-value block, so a token's output takes, per block, S = 256 S1 + S0 of
+// its two digit rows and one fused multiply-add of S by d_w d_x: four VALU
+// instructions per output and block, which bound it (64 MFMAs of 32 cycles
+// against 1,024 VALU instructions per wavefront and 64 tokens).  The block's
+// operand of a lane is the eight bytes of lane groups 2 h and 2 h + 1.
+// Measured against the expert kernel's items of 8 tokens (each tile read and
+// its three instructions per digit row and block repeated for every 8):
+// attention half of 200 tokens 180 -> 113 us, of 2,048 tokens 1,386 -> 668.
+struct XgQ80 {
+    static constexpr int TILE = Q80_TILE, TLDS = Q80_TILE, ASTAGES = 2, ALOADS = 6;
+    static constexpr bool MIN = false, PER32 = true;
+    struct Raw {
+        v4i w[8];
+        uint4 d;                         // the row's eight f16 scales
+    };
+    struct Ops {
+        v4i w[8];
+        float d[8];
+    };
+    __device__ static void read(Raw &t, const uint8_t *tile, int r16, int h)
+    {
+        const uint8_t *p = tile + r16 * 16;
+        t.d = *reinterpret_cast<const uint4 *>(p);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const uint8_t *q = p + (1 + 8 * h + (j >> 1)) * 256 + 8 * (j & 1);
+            const uint2 a = *reinterpret_cast<const uint2 *>(q), b = *reinterpret_cast<const uint2 *>(q + 1024);
+            t.w[j] = (v4i){(int)a.x, (int)a.y, (int)b.x, (int)b.y};
+        }
+    }
+    __device__ static void pin(Raw &t)
+    {
+        asm volatile("" : "+v"(t.d.x), "+v"(t.d.y), "+v"(t.d.z), "+v"(t.d.w));
+#pragma unroll
+        for (int j = 0; j < 8; j++) asm volatile("" : "+v"(t.w[j]));
+    }
+    __device__ static void fold(const Raw &t, int, Ops &f)
+    {
+        const uint32_t dw[4] = {t.d.x, t.d.y, t.d.z, t.d.w};
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            f.w[j] = t.w[j];
+            f.d[j] = h16f(j & 1 ? dw[j >> 1] >> 16 : dw[j >> 1] & 0xffffu);
         }
     }
 };
@@ -412,7 +462,7 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
         const ActI8 &A = DOWN ? (C.shared ? job.ahs : job.ah) : (C.shared ? job.axs : job.ax);
         aqb = reinterpret_cast<const uint8_t *>(A.q) + (size_t)sb0 * 256;
         absb = reinterpret_cast<const uint8_t *>(A.bs) + (size_t)sb0 * 32;
-        adb = reinterpret_cast<const uint8_t *>(A.d) + (size_t)sb0 * 4;
+        adb = reinterpret_cast<const uint8_t *>(A.d) + (size_t)sb0 * (F::PER32 ? 32 : 4);
         // (the lane through an empty asm: its rows and units are formed here,
         // once per item, and not held in registers across the steps)
         int ln = lane;
@@ -422,7 +472,8 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
         for (int j = 0; j < 4; j++)
             aqo[j] = (uint32_t)xg_arow<DOWN, MERGE>(C, pids, N, K, wave, 4 * j + (ln >> 4)) * (uint32_t)Kin + u;
         abso = ((uint32_t)xg_arow<DOWN, MERGE>(C, pids, N, K, wave, (ln >> 1) & 15) * (uint32_t)(Kin / 16) + (ln & 1) * 8) * 2;
-        ado = (uint32_t)xg_arow<DOWN, MERGE>(C, pids, N, K, wave, ln & 15) * (uint32_t)(Kin / 256) * 4;
+        ado = (uint32_t)xg_arow<DOWN, MERGE>(C, pids, N, K, wave, ln & 15) * (uint32_t)(Kin / 256);
+        ado = F::PER32 ? (8 * ado + (ln >> 4)) * 4 : 4 * ado;
     };
     // the weight cursor's super-block to the wavefront's stage ws; on to the next
     auto issue_w = [&](int ws) {
@@ -451,17 +502,24 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
             xg_lds16(aqb, aqo[j], blk + 1024 * q + 64 * (q >> 1));
         }
         if (F::MIN && lane < 32) xg_lds16(absb, abso, blk + XG_ABS + 512 * (wave & 1));
-        if (lane < 16) xg_lds4(adb, ado, blk + XG_AD + 64 * (wave & 1));
+        if (F::PER32) {
+            // scales [8 blocks][16 rows], four blocks a load, in place of the sums
+            xg_lds4(adb, ado, blk + XG_ABS + 512 * (wave & 1));
+            xg_lds4(adb + 16, ado, blk + XG_ABS + 512 * (wave & 1) + 256);
+        } else if (lane < 16) {
+            xg_lds4(adb, ado, blk + XG_AD + 64 * (wave & 1));
+        }
         aqb += 256;
         absb += 32;
-        adb += 4;
+        adb += F::PER32 ? 32 : 4;
     };
     // this lane's operand addresses in a stage: row r32, unit 8 gp + 4 h + c
-    // (c's swizzle in the address, gp 128 bytes on)
+    // (c's swizzle in the address, gp 128 bytes on); PER32: units 8 h + c and,
+    // 64 bytes on, 8 h + 4 + c
     uint32_t ao[4];
 #pragma unroll
     for (int c = 0; c < 4; c++)
-        ao[c] = 1024 * (r32 >> 2) + 64 * (r32 >> 3) + 256 * (r32 & 3) + 64 * h + 16 * (c ^ (r32 & 3));
+        ao[c] = 1024 * (r32 >> 2) + 64 * (r32 >> 3) + 256 * (r32 & 3) + (F::PER32 ? 128 : 64) * h + 16 * (c ^ (r32 & 3));
     const uint8_t *wrd = &SW[wave][0][((lane >> 4) & 1) * F::TLDS];
 
     weights_of(I, slice);
@@ -538,7 +596,73 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
                 auto read_a = [&](int b, int i) __attribute__((always_inline)) -> v4i {
                     return *reinterpret_cast<const v4i *>(st + b * XG_ABLK + ao[i & 3] + 128 * (i >> 2));
                 };
-                if constexpr (MERGE) {
+                if constexpr (F::PER32) {
+                    static_assert(!F::PER32 || (MERGE && DOWN), "Q8_0: projections");
+                    // block b's operand of 32-value block j
+                    auto read_q = [&](int b, int j) __attribute__((always_inline)) -> v4i {
+                        const uint8_t *q = st + b * XG_ABLK + ao[j >> 1] + 8 * (j & 1);
+                        const uint2 u = *reinterpret_cast<const uint2 *>(q), v = *reinterpret_cast<const uint2 *>(q + 64);
+                        return (v4i){(int)u.x, (int)u.y, (int)v.x, (int)v.y};
+                    };
+                    // scales of block j, activation rows 8 i + 4 h .. + 3
+                    auto read_dx = [&](int b, int j, int i) __attribute__((always_inline)) -> f4 {
+                        return *reinterpret_cast<const f4 *>(st + b * XG_ABLK + XG_ABS + 512 * (i >> 1) + 64 * j +
+                                                             32 * (i & 1) + 16 * h);
+                    };
+                    // (token block, 32-value block) n = 8 c + j: the next pair's
+                    // MFMAs go out before this pair's scale products
+                    constexpr int T = 8 * NB;
+                    if constexpr (NB > 0) {
+                        v4i x1[2], x0[2];
+                        v16i p1[2], p0[2];
+                        x1[0] = read_q(0, 0);
+                        x0[0] = read_q(1, 0);
+                        x1[1] = read_q(0, 1);
+                        x0[1] = read_q(1, 1);
+                        p1[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x1[0], f.w[0], (v16i)(0), 0, 0, 0);
+                        p0[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x0[0], f.w[0], (v16i)(0), 0, 0, 0);
+#pragma unroll
+                        for (int n = 0; n < T; n++) {
+                            const int c = n >> 3, j = n & 7, u = n & 1;
+                            __builtin_amdgcn_sched_barrier(0);
+                            f4 dx[4];
+#pragma unroll
+                            for (int i = 0; i < 4; i++) dx[i] = read_dx(2 * c + 1, j, i);
+                            if (n + 2 < T) {
+                                x1[u] = read_q(2 * ((n + 2) >> 3), (n + 2) & 7);
+                                x0[u] = read_q(2 * ((n + 2) >> 3) + 1, (n + 2) & 7);
+                            }
+                            if (n + 1 < T) {
+                                p1[u ^ 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x1[u ^ 1], f.w[(n + 1) & 7], (v16i)(0), 0, 0, 0);
+                                p0[u ^ 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x0[u ^ 1], f.w[(n + 1) & 7], (v16i)(0), 0, 0, 0);
+                            }
+#pragma unroll
+                            for (int i = 0; i < 16; i++)
+                                acc[c][i] = __builtin_fmaf((float)(256 * p1[u][i] + p0[u][i]), f.d[j] * dx[i >> 2][i & 3], acc[c][i]);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if constexpr (HALF) {
+                        v4i x[2];
+                        v16i p[2];
+                        x[0] = read_q(2 * NB, 0);
+                        x[1] = read_q(2 * NB, 1);
+                        p[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[0], f.w[0], (v16i)(0), 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            const int u = j & 1;
+                            __builtin_amdgcn_sched_barrier(0);
+                            const f4 dx[2] = {read_dx(2 * NB, j, 2), read_dx(2 * NB, j, 3)};
+                            if (j + 2 < 8) x[u] = read_q(2 * NB, j + 2);
+                            if (j + 1 < 8)
+                                p[u ^ 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[u ^ 1], f.w[(j + 1) & 7], (v16i)(0), 0, 0, 0);
+#pragma unroll
+                            for (int i = 0; i < 8; i++)
+                                acc[NB][i] = __builtin_fmaf((float)(256 * p[u][i] + p[u][i + 8]), f.d[j] * dx[i >> 2][i & 3], acc[NB][i]);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                } else if constexpr (MERGE) {
                     // block c: 32 tokens, their a1 rows in stage block 2 c, a0
                     // rows in 2 c + 1; the four digit products of a chunk, then
                     // one epilogue per token
@@ -802,7 +926,7 @@ hipError_t launch_expert_gemm_q4k(int phase, const MoeJob &job, hipStream_t s)
     const bool routed = job.eg.data || job.ed.data;
     const WTensor &wr = phase == 0 ? job.eg : job.ed, &ws = phase == 0 ? job.sg : job.sd;
     if ((routed && wr.type != DMOE_TYPE_Q4_K) || (!routed && !job.has_shared) ||
-        (job.has_shared && ws.type != DMOE_TYPE_Q4_K && (routed || ws.type != DMOE_TYPE_Q6_K)))
+        (job.has_shared && ws.type != DMOE_TYPE_Q4_K && (routed || (ws.type != DMOE_TYPE_Q6_K && ws.type != DMOE_TYPE_Q8_0))))
         return hipErrorInvalidValue;
     if (!expert_gemm_q4k_ok(job.H, job.FF, job.SF, job.has_shared) || job.wl.chunk != XG_CHUNK ||
         (routed && !job.wl.n_ec))
@@ -828,6 +952,11 @@ hipError_t launch_expert_gemm_q4k(int phase, const MoeJob &job, hipStream_t s)
     if (e != hipSuccess) return e;
     const int grid = ((n_cu + 7) / 8) * 8;
     const dim3 gd(grid), bd(XG_WAVES * 64);
+    if (ws.type == DMOE_TYPE_Q8_0) {
+        if (routed || phase == 0) return hipErrorInvalidValue;
+        hipLaunchKernelGGL((k_gemm_q<XgQ80, true, true>), gd, bd, 0, s, job);
+        return hipGetLastError();
+    }
     if (ws.type == DMOE_TYPE_Q6_K && !routed && phase == 1 && N <= XG_SCHUNK / 2) {
         hipLaunchKernelGGL((k_gemm_q<XgQ6K, true, true, true>), gd, bd, 0, s, job);
     } else if (ws.type == DMOE_TYPE_Q6_K && !routed) {

@@ -75,8 +75,8 @@ __global__ __launch_bounds__(NORM_THREADS) void k_residual_rmsnorm(float *__rest
 // with their producers and consumers folded in: the residual added is the sum
 // of a projection's KS reduction slices (in slice order, as k_proj_reduce
 // adds them), h may be read from one buffer and written to another, and the
-// normed row may leave as two int8 digit rows (ACT_SPLIT, prep_values, one
-// wavefront per super-block) for the next projection instead of (or beside)
+// normed row may leave as two int8 digit rows (ACT_SPLIT or ACT_SPLIT32,
+// prep_values, one wavefront per super-block) for the next projection instead of (or beside)
 // f32.  The row is staged in LDS between the sum and the outputs.  The sum
 // runs on the first NORM_THREADS threads in k_residual_rmsnorm's order; the
 // outputs use all NF_THREADS.
@@ -159,7 +159,8 @@ __global__ __launch_bounds__(NF_THREADS) void k_norm_fused(NormArgs a)
                 if (a.gain) o = o * a.gain[i];
                 v[c] = o;
             }
-            prep_values(v, a.act, ACT_SPLIT, row, a.rows, sb, nsb, s_v[w]);
+            // (no sums of 16: the operand with a scale per 32 values)
+            prep_values(v, a.act, a.act.bs ? ACT_SPLIT : ACT_SPLIT32, row, a.rows, sb, nsb, s_v[w]);
         }
     }
 }

@@ -13,7 +13,7 @@ from conftest import max_rel_err
 pytestmark = pytest.mark.gpu
 
 TOL = 5e-4
-WTYPES = [12, 14]
+WTYPES = [12, 14, 8]
 
 
 @pytest.mark.parametrize("wtype", WTYPES)
@@ -32,7 +32,24 @@ def test_head_units(ctx, O, wtype, N):
     head.free()
 
 
-@pytest.mark.parametrize("wtype", WTYPES)
+@pytest.mark.parametrize("N", [1, 7, 16, 17, 32])
+def test_head_q80_few_tokens(ctx, O, N):
+    """Q8_0 projections take the GEMM at any token count (half blocks, one
+    token), unless they are an LM head's."""
+    from dmoe import synth
+    H, V = 1024, 1280
+    print(f"case: LM head H={H} V={V} Q8_0 N={N}", flush=True)
+    w = synth.host_head(H, V, 8, 60 + N, O.quantize_rows)
+    h = (synth.normal(61 + N, synth.S_X, N * H).reshape(N, H) * 2).astype(np.float32)
+    head = ctx.head_upload(w)
+    lg = ctx.head_forward(head, h, 1e-6, logits=True)[2]
+    err = max_rel_err(lg, O.head_forward(w, h, 1e-6)[2])
+    print(f"  max rel err {err:.3e}", flush=True)
+    assert err <= TOL
+    head.free()
+
+
+@pytest.mark.parametrize("wtype", [12, 14])
 @pytest.mark.parametrize("N", [33, 64, 90, 129])
 def test_dense_units(ctx, O, wtype, N):
     from dmoe import synth
