@@ -336,6 +336,125 @@ __global__ __launch_bounds__(256) void k_front(FrontArgs a)
     }
 }
 
+// Many tokens: the same partials and the same butterfly on f32 MFMA.
+// v_mfma_f32_16x16x1_4b_f32 forms, in each of four blocks, C[r][c] <- fma(A[r],
+// B[c], C[r][c]) with one rounding and no flush of subnormals, so a block can
+// carry one of logits_wave's 64 chains for a 16 x 16 tile of outputs: block q
+// (the operands of lanes 16 q ..) holds partial l = 4 cg + q of chain group cg,
+// and the four MFMAs of a lane's float4 x[256 i + 4 l ..], W[256 i + 4 l ..]
+// are the steps j = 0 .. 3 of that chain.  One workgroup per 32 tokens x 32
+// experts: wavefront w runs chain groups w and w + 8 of the tile (2 x 2 MFMA
+// tiles), its operands of the next 256 values in flight.  Then the butterfly's
+// rounds in their order: 32 adds groups w and w + 8 in registers, 16, 8, 4 add
+// wavefronts w ^ 4, w ^ 2, w ^ 1 through LDS, 2 and 1 blocks q ^ 2, q ^ 1;
+// both partners of a round add the same two values, so one sum serves both.
+//
+// What bounds the logits of many tokens is what the CUs read from L2: a
+// wavefront's tile of 8 x 8 outputs reads 16 rows for 64 outputs, this tile 64
+// rows for 1,024 (2.1 GB against 0.5 GB at 2,048 tokens of 4,096 values and
+// 256 experts; the multiply-adds alone take about 30 us on either unit).
+// Measured at 4,096 values and 256 experts: the logits and two conversions of
+// 2,048 tokens 138 -> 80 + 29 us (two launches), the Q4_K layer of 2,048 / 1,024
+// / 777 tokens 1,012 -> 956, 582 -> 553, 615 -> 604 us.  Below 192 tiles too few
+// CUs have one: 512 tokens 385 -> 391, 256 tokens 268 -> 283 us, so those stay
+// on logits_wave.  (A second step of operands in flight changed nothing.)
+typedef float lm_f16v __attribute__((ext_vector_type(16)));
+constexpr int LM_T = 32, LM_E = 32, LM_WAVES = 8;
+constexpr long LM_MIN_TILES = 192;
+
+__global__ __launch_bounds__(LM_WAVES * 64) void k_logits_mfma(const float *__restrict__ W,
+                                                               const float *__restrict__ bias,
+                                                               const float *__restrict__ x, int N, int H, int E,
+                                                               RouteBufs rb)
+{
+    __shared__ float s_p[4][16][LM_WAVES][64];        // [MFMA tile][register][wavefront][lane]
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, q = lane >> 4;
+    // the expert tiles of one token tile run on one XCD (workgroup b on XCD b
+    // % 8): its rows of x come from that XCD's L2
+    const int ne = (E + LM_E - 1) / LM_E;
+    const int tt = (blockIdx.x >> 3) / ne * 8 + (blockIdx.x & 7), et = (blockIdx.x >> 3) % ne;
+    const int t0 = tt * LM_T, e0 = et * LM_E;
+    if (t0 >= N) return;
+    const float4 *xr[2], *wr[2];
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        xr[a] = reinterpret_cast<const float4 *>(x + (size_t)min(t0 + 16 * a + r16, N - 1) * H) + 4 * w + q;
+        wr[a] = reinterpret_cast<const float4 *>(W + (size_t)min(e0 + 16 * a + r16, E - 1) * H) + 4 * w + q;
+    }
+    // acc[chain group w + 8 c][token half a][expert half b]
+    lm_f16v acc[2][2][2];
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) acc[c][a][b] = (lm_f16v)(0.0f);
+    float4 xv[2][2][2], wv[2][2][2];                  // [set][c][row half]
+    const int steps = H / 256;
+    auto load = [&](int set, int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int a = 0; a < 2; a++) {
+                xv[set][c][a] = xr[a][i * 64 + 32 * c];
+                wv[set][c][a] = wr[a][i * 64 + 32 * c];
+            }
+    };
+    auto products = [&](int set) __attribute__((always_inline)) {
+        auto el = [](const float4 &v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; };
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int c = 0; c < 2; c++)
+#pragma unroll
+                for (int a = 0; a < 2; a++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++)
+                        acc[c][a][b] = __builtin_amdgcn_mfma_f32_16x16x1f32(el(xv[set][c][a], j), el(wv[set][c][b], j),
+                                                                            acc[c][a][b], 0, 0, 0);
+    };
+    load(0, 0);
+    for (int i = 0; i + 2 <= steps; i += 2) {
+        load(1, i + 1);
+        products(0);
+        load(0, min(i + 2, steps - 1));
+        products(1);
+    }
+    if (steps & 1) products(0);
+    // register 4 q + k of a tile: block q, token 4 (lane / 16) + k, expert lane % 16
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int k = 0; k < 16; k++) s_p[2 * a + b][k][w][lane] = acc[0][a][b][k] + acc[1][a][b][k];
+    __syncthreads();
+    // wavefront w: tile w / 2, registers k = 2 (w % 2) + {0, 1} of every block
+    const int tile = w >> 1;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int k = 2 * (w & 1) + u;
+        float v[4];
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            float p[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) p[i] = s_p[tile][4 * b + k][i][lane];
+            v[b] = ((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]));
+        }
+        const float logit = (v[0] + v[2]) + (v[1] + v[3]);
+        const int t = t0 + 16 * (tile >> 1) + 4 * q + k, e = e0 + 16 * (tile & 1) + r16;
+        if (t < N && e < E) {
+            const size_t o = (size_t)t * E + e;
+            const float p = sigmoid_f32(logit);
+            rb.logits[o] = logit;
+            rb.probs[o] = p;
+            rb.sel[o] = bias ? p + bias[e] : p;
+        }
+    }
+}
+
 hipError_t launch_front(const float *W, const float *bias, const float *x, int N, int H, int E,
                         const RouteBufs &rb, const PrepJob *jobs, int njobs, hipStream_t s)
 {
@@ -347,6 +466,14 @@ hipError_t launch_front(const float *W, const float *bias, const float *x, int N
     a.H = H;
     a.E = E;
     a.rb = rb;
+    // tiles of 32 x 32 outputs once they fill three quarters of the CUs
+    const int ntt = (N + LM_T - 1) / LM_T, net = (E + LM_E - 1) / LM_E;
+    if ((long)ntt * net >= LM_MIN_TILES && H % 256 == 0) {
+        hipLaunchKernelGGL(k_logits_mfma, dim3((ntt + 7) / 8 * 8 * net), dim3(LM_WAVES * 64), 0, s, W, bias, x, N, H, E,
+                           rb);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess || njobs == 0 ? e : launch_prep(jobs, njobs, s);
+    }
     a.wide = N >= 256;
     a.small = !a.wide && (H == 256 || H == 512 || H == 1024 || H == 2048 || H == LS_MAXK * 256);
     a.logit_blocks = a.small ? small_tiles(N, E) : (logit_waves(N, E, a.wide) + 3) / 4;
