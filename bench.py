@@ -133,7 +133,7 @@ def uses_tile_kernels(cfg):
 def uses_q4k_gemm(cfg):
     """Whether the library runs cfg's Q4_K expert products on its grouped
     GEMM (k_expert_gemm.hip): the rule of use_q4k_gemm in dmoe_api.cpp for
-    the flash shapes (64 or more pairs per expert averaged over all experts,
+    the flash shapes (32 or more pairs per expert averaged over all experts,
     N k / E), DMOE_EXPERT_GEMM overriding it and DMOE_EXPERT_TILE turning it
     off."""
     import dmoe
@@ -144,7 +144,7 @@ def uses_q4k_gemm(cfg):
         return env == "1"
     if os.environ.get("DMOE_EXPERT_TILE") in ("0", "1") or os.environ.get("DMOE_Q4K_COLUMN_BLOCKS"):
         return False
-    return cfg.n_tokens * cfg.top_k // cfg.n_experts >= 64
+    return cfg.n_tokens * cfg.top_k // cfg.n_experts >= 32
 
 
 def bench_layer(a, cfg, steps, warmup, copies, cpu_seconds, cpu_tokens=None):
@@ -256,7 +256,7 @@ def bench_layer(a, cfg, steps, warmup, copies, cpu_seconds, cpu_tokens=None):
             def act_row(n):
                 return 2 * n
         if uses_q4k_gemm(cfg):
-            dom_kernel = "dmoe::k_gemm_q4k<false>"
+            dom_kernel = "dmoe::k_gemm_q<dmoe::XgQ4K, false, false, false>"
             h_bytes = P * FF * 4 + N * SF * 4
         elif fmt and tile:
             dom_kernel = f"dmoe::k_gu_rr<dmoe::{fmt}>"

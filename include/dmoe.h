@@ -255,8 +255,8 @@ void dmoe_layer_free(dmoe_layer *layer);
  *   DMOE_PATH_Q80_MFMA  Q8_0 routed + shared experts on int8 MFMA tiles
  *   DMOE_PATH_F16_GEMM  F16 experts on the f16 MFMA grouped GEMM
  *   DMOE_PATH_Q6K_MFMA  Q6_K dense MLP, step-tail LM head or attention
- *                       projections on int8 MFMA tiles (few-token kernel, in
- *                       chunks of 32 tokens)
+ *                       projections on int8 MFMA tiles (the few-token kernel
+ *                       or the grouped GEMM, by tokens)
  *   DMOE_PATH_GEMV      every other type / shape mix (F32 experts; Q6_K
  *                       routed or shared experts; widths
  *                       that are not whole MFMA work items; a shared expert
