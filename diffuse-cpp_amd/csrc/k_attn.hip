@@ -34,6 +34,15 @@ namespace dmoe {
 typedef float f4v __attribute__((ext_vector_type(4)));
 
 constexpr int QR_THREADS = 256;
+// From QR_MANY (token, head) rows on a wavefront takes QR_HEADS heads of its
+// token: it waits on its loads (4 bytes per lane, two per row of 128) and then
+// on the angle's chain, and with four rows loaded at once and one angle for all
+// the launch of 2,048 tokens of 40 heads leaves the attention half at 580 us
+// against 591.  Fewer rows need the wavefronts: 777 tokens 243 us either way,
+// 256 tokens 105 against 102 (eight heads: 581, 251, 112 us); one head per
+// wavefront by that kernel takes 48.0 us at 32 tokens against 47.3.
+constexpr int QR_HEADS = 4;
+constexpr long QR_MANY = 65536;
 
 __global__ __launch_bounds__(QR_THREADS) void k_qk_rope(const float *__restrict__ qkv, int ks, size_t kstride,
                                                         const float *__restrict__ qn,
@@ -93,13 +102,116 @@ __global__ __launch_bounds__(QR_THREADS) void k_qk_rope(const float *__restrict_
     for (int d = lane; d < HD; d += 64) dst[d] = x[d];
 }
 
+// The same, QR_HEADS heads of one token per wavefront, their rows all loaded
+// before the first is used and one rotation for all (the same operations in
+// the same order).
+__global__ __launch_bounds__(QR_THREADS) void k_qk_rope_heads(const float *__restrict__ qkv, int ks, size_t kstride,
+                                                              const float *__restrict__ qn,
+                                                              const float *__restrict__ kn, AttnDims a,
+                                                              float *__restrict__ Qh, float *__restrict__ Kh,
+                                                              float *__restrict__ Vh)
+{
+    constexpr int HB = QR_HEADS;
+    __shared__ float s_x[QR_THREADS / 64][256];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int heads = a.nh + 2 * a.nkv, groups = (heads + HB - 1) / HB;
+    const int item = blockIdx.x * (QR_THREADS / 64) + w;
+    if (item >= a.n * groups) return;
+    const int t = item / groups, h0 = (item % groups) * HB;
+    const int HD = a.hd, QKV = (a.nh + 2 * a.nkv) * HD;
+    const float *row = qkv + (size_t)t * QKV;
+    float *x = s_x[w];
+    // the fused projection's rows: the sum of its ks reduction slices, in order
+    float v[HB][4];
+#pragma unroll
+    for (int b = 0; b < HB; b++) {
+        const float *src = row + (size_t)min(h0 + b, heads - 1) * HD;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (64 * i < HD) v[b][i] = lane + 64 * i < HD ? src[lane + 64 * i] : 0.0f;
+    }
+    for (int k = 1; k < ks; k++)
+#pragma unroll
+        for (int b = 0; b < HB; b++) {
+            const float *src = row + (size_t)k * kstride + (size_t)min(h0 + b, heads - 1) * HD;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (64 * i < HD && lane + 64 * i < HD) v[b][i] = v[b][i] + src[lane + 64 * i];
+        }
+    // the token's rotation, the same for all its heads
+    const int half = a.rd / 2;
+    float c = 1.0f, sn = 0.0f;
+    if (lane < half && h0 < a.nh + a.nkv) {
+        float theta = (float)t;
+        for (int i = 0; i < lane; i++) theta *= a.theta_scale;
+        c = cosf(theta);
+        sn = sinf(theta);
+    }
+#pragma unroll
+    for (int b = 0; b < HB; b++) {
+        const int hh = h0 + b;
+        if (hh >= heads) break;
+        if (hh < a.nh + a.nkv) {
+            if (a.qk_norm) {
+                double acc = 0.0;
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (64 * i < HD && lane + 64 * i < HD) acc += (double)(v[b][i] * v[b][i]);
+#pragma unroll
+                for (int m = 32; m >= 1; m >>= 1) acc += __shfl_xor(acc, m, 64);
+                const float mean = (float)(acc / (double)HD);
+                const float scale = 1.0f / sqrtf(mean + a.eps);
+                const float *nw = hh < a.nh ? qn : kn;
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (64 * i < HD && lane + 64 * i < HD) v[b][i] = (v[b][i] * scale) * nw[lane + 64 * i];
+            }
+            // pairs (ic, ic + rd / 2) through LDS
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (64 * i < HD && lane + 64 * i < HD) x[lane + 64 * i] = v[b][i];
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            if (lane < half) {
+                const float x0 = x[lane], x1 = x[lane + half];
+                x[lane] = x0 * c - x1 * sn;
+                x[lane + half] = x0 * sn + x1 * c;
+            }
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (64 * i < HD && lane + 64 * i < HD) v[b][i] = x[lane + 64 * i];
+        }
+        float *dst;
+        if (hh < a.nh)
+            dst = Qh + ((size_t)hh * a.n + t) * HD;
+        else if (hh < a.nh + a.nkv)
+            dst = Kh + ((size_t)(hh - a.nh) * a.n + t) * HD;
+        else
+            dst = Vh + ((size_t)(hh - a.nh - a.nkv) * a.n + t) * HD;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (64 * i < HD && lane + 64 * i < HD) dst[lane + 64 * i] = v[b][i];
+    }
+}
+
 hipError_t launch_qk_rope(const float *qkv, int ks, size_t kstride, const float *qn, const float *kn,
                           const AttnDims &a, float *Qh, float *Kh, float *Vh, hipStream_t s)
 {
     if (a.hd <= 0 || a.hd > 256 || a.rd > a.hd || a.rd % 2 || a.rd / 2 > 64 || ks < 1) return hipErrorInvalidValue;
-    const int items = a.n * (a.nh + 2 * a.nkv);
-    hipLaunchKernelGGL(k_qk_rope, dim3((items + 3) / 4), dim3(QR_THREADS), 0, s, qkv, ks, kstride, qn, kn, a, Qh,
-                       Kh, Vh);
+    const int heads = a.nh + 2 * a.nkv;
+    if ((long)a.n * heads >= QR_MANY) {
+        const int items = a.n * ((heads + QR_HEADS - 1) / QR_HEADS);
+        hipLaunchKernelGGL(k_qk_rope_heads, dim3((items + 3) / 4), dim3(QR_THREADS), 0, s, qkv, ks, kstride, qn, kn,
+                           a, Qh, Kh, Vh);
+    } else {
+        const int items = a.n * heads;
+        hipLaunchKernelGGL(k_qk_rope, dim3((items + 3) / 4), dim3(QR_THREADS), 0, s, qkv, ks, kstride, qn, kn, a, Qh,
+                           Kh, Vh);
+    }
     return hipGetLastError();
 }
 
