@@ -306,8 +306,9 @@ int expert_tile_chunk(int32_t type);
 hipError_t launch_expert_tile(int phase, const MoeJob &job, hipStream_t s);
 // Q4_K expert products as a grouped int8-MFMA GEMM for many pairs per expert
 // (k_expert_gemm.hip): units of up to 128 pairs (the work list's chunk) or
-// 64 shared tokens, a step's weights and activations streamed through LDS
-// together; h / hs and ye / ys as with the tile kernels.
+// 64 shared tokens, weights and activations streamed through LDS; h / hs and ye
+// / ys as with the tile kernels.  Without routed weights (a projection, the
+// dense MLP) also Q6_K, and Q8_0 for phase 1.
 constexpr int EXPERT_GEMM_CHUNK = 128;
 bool expert_gemm_q4k_ok(int H, int FF, int SF, bool shared);
 hipError_t launch_expert_gemm_q4k(int phase, const MoeJob &job, hipStream_t s);

@@ -5,6 +5,8 @@
 //     summation order, with probs = sigmoid(L) (:204) and the selection score
 //     sel = probs + bias (:207-210) computed by the lane that owns each logit;
 //   * up to two conversions of x into the MFMA operand layout of k_expert.hip.
+// For many tokens the logits are a launch of f32 MFMA tiles (k_logits_mfma)
+// and the conversions one of their own.
 //
 // The conversions themselves (Q8_K for the routed experts, two int8 digits
 // for the shared expert) are in dmoe_prep.h.
