@@ -1018,7 +1018,6 @@ int finish_layer(dmoe_ctx *ctx, dmoe_layer *L, const dmoe_hparams *hp, const dmo
 // ---------------------------------------------------------------------------
 // Dense MLP (src/diffuse-moe-graph.cpp:181-187): the shared expert's kernels
 // with an empty routed work list; the down launch writes y directly.
-enum DensePath { DP_GEMV = 0, DP_Q4K, DP_Q80, DP_F16, DP_Q6K };
 
 int dense_path(int32_t type, int H, int FF)
 {
@@ -1095,21 +1094,11 @@ struct DenseWs {
     float *part_gu, *part_d;             // slice sums of the few-token Q4_K projections
 };
 
-// Few tokens of a Q4_K or Q6_K dense MLP: gate and up as one two-matrix
-// projection, h formed and converted from their slice sums, down as a
-// projection.  Q6_K weights take every token count this way, in chunks of up
-// to PROJ_MAX_TOKENS tokens (dense_chunk).
-bool dense_few(int path, int H, int FF, int N)
+// The compute units the routes are planned for (without a device: a whole chip).
+int plan_cus()
 {
-    return (path == DP_Q4K || path == DP_Q6K) && proj_ok(FF, H, N) && proj_ok(H, FF, N) && FF % 256 == 0;
-}
-
-int dense_gemm_slices(const KernelSwitches &sw, int path, int H, int FF, int N);
-
-// (Q6_K shapes that the GEMM does not take)
-int dense_chunk(const KernelSwitches &sw, int path, int H, int FF, int N)
-{
-    return path == DP_Q6K && !dense_gemm_slices(sw, path, H, FF, N) ? std::min(N, PROJ_MAX_TOKENS) : N;
+    int n_cu = 0;
+    return device_cu_count(&n_cu) == hipSuccess ? n_cu : 256;
 }
 
 // Slice-sum floats the few-token projection of R x K (M matrices) needs at
@@ -1164,13 +1153,14 @@ size_t plan_dense(const KernelSwitches &sw, const dmoe_layer *L, int N, bool hos
     case DP_Q4K:
     case DP_Q6K: {
         // Q6_K in chunks: workspace for one, reused chunk after chunk
-        const int n = dense_chunk(sw, path, H, FF, N);
+        const ProjRoute r = dense_route(sw, path, H, FF, N, plan_cus());
+        const int n = r.chunk, ks = r.gemm_ks;
         t.axs = take_act(take, n, H, true);
         t.ahs = take_act(take, n, FF, true);
-        if (dense_few(path, H, FF, n)) {
+        if (r.few) {
             t.part_gu = (float *)take(proj_partial_max(FF, H, 2, n, false) * 4);
             if (const size_t pd = proj_partial_max(H, FF, 1, n, true)) t.part_d = (float *)take(pd * 4);
-        } else if (const int ks = dense_gemm_slices(sw, path, H, FF, N)) {
+        } else if (ks) {
             // the grouped GEMM: f32 h, the down launch's slices
             t.hs = (float *)take((size_t)N * FF * 4);
             if (ks > 1) t.part_d = (float *)take((size_t)ks * N * H * 4);
@@ -1223,11 +1213,12 @@ int enqueue_dense(dmoe_ctx *ctx, const dmoe_layer *L, const DenseWs &w, const fl
         STAGE(ST_SH_DOWN, launch_down_shared(L->sd, w.hs, N, FF, H, y, s));
         return DMOE_OK;
     }
-    if (dense_few(path, H, FF, dense_chunk(ctx->sw, path, H, FF, N))) {
+    const ProjRoute r = dense_route(ctx->sw, path, H, FF, N, plan_cus());
+    if (r.few) {
         // gate and up: one launch over both matrices, h from their slices;
         // tokens t0 .. t0 + n - 1 at a time (every token at once, or Q6_K chunks)
         const bool q6 = path == DP_Q6K;
-        const int nc = dense_chunk(ctx->sw, path, H, FF, N);
+        const int nc = r.chunk;
         for (int t0 = 0; t0 < N; t0 += nc) {
             const int n = std::min(nc, N - t0);
             ProjJob gu{};
@@ -1261,7 +1252,7 @@ int enqueue_dense(dmoe_ctx *ctx, const dmoe_layer *L, const DenseWs &w, const fl
         }
         return DMOE_OK;
     }
-    if (const int ks = dense_gemm_slices(ctx->sw, path, H, FF, N)) {
+    if (const int ks = r.gemm_ks) {
         // many tokens of Q4_K or Q6_K: the grouped GEMM's gate/up and down launches
         // over shared units (no routed work list), h converted between them,
         // the down reduction in slices added in order
@@ -1319,6 +1310,7 @@ int enqueue_dense(dmoe_ctx *ctx, const dmoe_layer *L, const DenseWs &w, const fl
         return DMOE_OK;
     }
     const bool q8 = path == DP_Q80;
+    if (!q8 && path != DP_Q4K) return set_err(ctx, DMOE_ERR_UNSUPPORTED_TYPE, "dense: no kernel for type %d", L->sg.type);
     wl.chunk = EXPERT_CHUNK;
     MoeJob job{};
     job.sg = L->sg;
@@ -1360,10 +1352,6 @@ int head_path(int32_t type, int V, int H)
     return DP_GEMV;
 }
 
-// Output rows up to which a few-token Q4_K projection runs one workgroup per
-// 16 rows (k_down_rows); above it (the LM head) the expert kernel's items.
-constexpr int PROJ_ROWS_MAX = 32768;
-
 // One projection y [N][rows] = W x with W's F32 semantics (x [N][K] f32):
 // the shared-down product of the expert kernels (Q4_K / Q8_0 on int8 digits,
 // F16 on hi / lo pairs) or the GEMV kernel.
@@ -1372,114 +1360,29 @@ struct ProjWs {
     ActI8 act;                           // split x (int8 paths)
     uint16_t *x16;                       // hi / lo f16 x (F16 path)
     float *part;                         // slice sums of the few-token Q4_K projection
+    ProjRoute route;                     // what the workspace is planned for and the launches take
 };
-
-// Q4_K, Q6_K and Q8_0 projections of proj_gemm_min_tokens or more tokens run on the
-// grouped GEMM's down launch (k_expert_gemm.hip) with shared units only: 64 tokens
-// (128 digit rows) per unit, 256 output rows per item, the reduction split
-// into slices of 2 or more super-blocks, as many as minimise the static
-// schedule's rounds x steps plus the slices' own traffic.  Returns the slice
-// count, 0 where the GEMM does not take the shape.
-constexpr int PROJ_GEMM_MIN_TOKENS = 33;
-
-// Q6_K matrices of an LM head's rows take the GEMM (in units of 32 tokens)
-// from 17 tokens on: at 157,184 x 4,096 rows 16 / 17 / 24 / 32 tokens 145 / 167
-// / 172 / 177 us against 140 / 174 / 177 / 217 on the few-token kernel, whose
-// work per weight grows by the eight tokens.  A few thousand rows fill too few
-// of the GEMM's 256-row items.
-constexpr int PROJ_GEMM_MIN_TOKENS_Q6K_HEAD = 17;
-
-// Q8_0 projections have no few-token kernel of their own: against the expert
-// kernel's items of 8 tokens the GEMM takes the attention half of 1 / 8 / 20
-// tokens from 95 / 98 / 99 us to 46 / 49 / 53, and an LM head of 16 / 32 tokens
-// from 233 / 468 us to 160 / 194; one item of the expert kernel covers a head
-// of up to 8 tokens (128 / 133 us at 1 / 8 tokens against 137 / 148).
-constexpr int PROJ_GEMM_MIN_TOKENS_Q80 = 1, PROJ_GEMM_MIN_TOKENS_Q80_HEAD = 9;
-
-int proj_gemm_min_tokens(int path, int rows)
-{
-    if (path == DP_Q80) return rows > PROJ_ROWS_MAX ? PROJ_GEMM_MIN_TOKENS_Q80_HEAD : PROJ_GEMM_MIN_TOKENS_Q80;
-    return path == DP_Q6K && rows > PROJ_ROWS_MAX ? PROJ_GEMM_MIN_TOKENS_Q6K_HEAD : PROJ_GEMM_MIN_TOKENS;
-}
-
-int proj_gemm_slices(const KernelSwitches &sw, int path, int rows, int K, int N)
-{
-    if ((path != DP_Q4K && path != DP_Q6K && path != DP_Q80) || sw.proj_gemm == 0 ||
-        (sw.proj_gemm < 0 && N < proj_gemm_min_tokens(path, rows)) ||
-        !expert_gemm_q4k_ok(rows, K, K, true) || 2L * N * K >= (1L << 31))
-        return 0;
-    int n_cu = 0;
-    if (device_cu_count(&n_cu) != hipSuccess || n_cu <= 0) n_cu = 256;
-    const long items = (long)((N + 63) / 64) * (rows / 256);
-    const int nsb = K / 256;
-    const long grid = (n_cu + 7) / 8 * 8;
-    // rounds of the static schedule x super-blocks per item at ~4.5 us per
-    // step, plus the slices written and read again at ~4 TB/s
-    int best = 1;
-    double best_us = 0.0;
-    for (int ks = 1; ks <= 16; ks *= 2) {
-        if (nsb % ks || (ks > 1 && nsb / ks < 2)) continue;
-        const long rounds = (items * ks + grid - 1) / grid;
-        double us = 4.5 * (double)(rounds * (nsb / ks));
-        if (ks > 1) us += (double)ks * N * rows * 8 / 4e6;
-        if (ks == 1 || us < best_us) {
-            best = ks;
-            best_us = us;
-        }
-    }
-    return best;
-}
-
-// Tokens per launch of a projection: every token, or, for Q6_K shapes that the
-// GEMM does not take, chunks of up to PROJ_MAX_TOKENS of the few-token kernel.
-int proj_chunk(const KernelSwitches &sw, int path, int rows, int K, int N)
-{
-    return path == DP_Q6K && !proj_gemm_slices(sw, path, rows, K, N) ? std::min(N, PROJ_MAX_TOKENS) : N;
-}
-
-// The dense MLP past the few-token kernels on the same GEMM (gate/up, then
-// down in proj_gemm_slices slices): 0 where it does not take the shape.
-int dense_gemm_slices(const KernelSwitches &sw, int path, int H, int FF, int N)
-{
-    if (path == DP_Q80 || 2L * N * H >= (1L << 31)) return 0;
-    return proj_gemm_slices(sw, path, H, FF, N);
-}
-
-bool proj_few(const KernelSwitches &sw, int path, int rows, int K, int N);
 
 template <class Take>
 ProjWs plan_proj(const KernelSwitches &sw, int path, int N, int K, int rows, Take &&take)
 {
     ProjWs p{};
     p.n_ec = (int32_t *)take(4);
+    p.route = proj_route(sw, path, rows, K, N, plan_cus());
+    const int n = p.route.chunk, ks = p.route.gemm_ks;
     switch (path) {
     case DP_Q4K:
-    case DP_Q6K: {
-        const int n = proj_chunk(sw, path, rows, K, N);
+    case DP_Q6K:
         p.act = take_act(take, n, K, true);
-        if (proj_few(sw, path, rows, K, n)) {
+        if (p.route.few)
             if (const size_t pf = proj_partial_max(rows, K, 1, n, true)) p.part = (float *)take(pf * 4);
-        } else if (const int ks = proj_gemm_slices(sw, path, rows, K, N); ks > 1) {
-            p.part = (float *)take((size_t)ks * N * rows * 4);
-        }
         break;
-    }
-    case DP_Q80:
-        p.act = take_act(take, N, K, true, true);
-        if (const int ks = proj_gemm_slices(sw, path, rows, K, N); ks > 1) p.part = (float *)take((size_t)ks * N * rows * 4);
-        break;
+    case DP_Q80: p.act = take_act(take, N, K, true, true); break;
     case DP_F16: p.x16 = (uint16_t *)take((size_t)2 * N * K * 2); break;
     default: break;
     }
+    if (ks > 1) p.part = (float *)take((size_t)ks * N * rows * 4);
     return p;
-}
-
-// Few tokens of Q4_K or Q6_K weights: k_proj.hip on x already converted to
-// p.act.
-bool proj_few(const KernelSwitches &sw, int path, int rows, int K, int N)
-{
-    if ((path != DP_Q4K && path != DP_Q6K) || !proj_ok(rows, K, N)) return false;
-    return N < proj_gemm_min_tokens(path, rows) || !proj_gemm_slices(sw, path, rows, K, N);
 }
 
 // y [N][rows] = W x from p.act: 128 T-row tiles x reduction slices over every
@@ -1513,11 +1416,12 @@ int enqueue_proj_few(dmoe_ctx *ctx, bool prof, int st_prod, const WTensor &W, in
 }
 
 // y [N][rows] = W x from p.act on the grouped GEMM's down launch over
-// shared units (no routed work list), in ks reduction slices; with ks_out the
+// shared units (no routed work list), in the route's reduction slices; with ks_out the
 // slices are left to the consumer as in enqueue_proj_few, else added into y.
-int enqueue_proj_gemm(dmoe_ctx *ctx, bool prof, int st_prod, const WTensor &W, int rows, int K, int N, int ks,
+int enqueue_proj_gemm(dmoe_ctx *ctx, bool prof, int st_prod, const WTensor &W, int rows, int K, int N,
                       const ProjWs &p, float *y, int *ks_out, const float **src_out, hipStream_t s)
 {
+    const int ks = p.route.gemm_ks;
 #define STAGE(id, call) LAUNCH_TRY(ctx, stage(ctx, prof, id, s, [&] { return call; }))
     MoeJob job{};
     job.sd = W;
@@ -1542,22 +1446,19 @@ int enqueue_proj_gemm(dmoe_ctx *ctx, bool prof, int st_prod, const WTensor &W, i
     return DMOE_OK;
 }
 
-// Projections that take p.act's digits from the caller (k_norm_fused writes
-// them beside its RMSNorm): the few-token kernel or, for many tokens of Q4_K,
-// the GEMM (*gemm_ks its slice count, else 0).
-bool proj_takes_digits(const KernelSwitches &sw, int path, int rows, int K, int N, int *gemm_ks)
+// Projections that take p.act's digits of all tokens from the caller
+// (k_norm_fused writes them beside its RMSNorm): the few-token kernel in one
+// launch, or the GEMM.
+bool proj_takes_digits(const ProjWs &p, int N)
 {
-    *gemm_ks = 0;
-    if (proj_few(sw, path, rows, K, N)) return true;
-    *gemm_ks = proj_gemm_slices(sw, path, rows, K, N);
-    return *gemm_ks > 0;
+    return p.route.gemm_ks > 0 || (p.route.few && p.route.chunk == N);
 }
 
-int enqueue_proj_digits(dmoe_ctx *ctx, bool prof, int st_prod, const WTensor &W, int rows, int K, int N, int gemm_ks,
+int enqueue_proj_digits(dmoe_ctx *ctx, bool prof, int st_prod, const WTensor &W, int rows, int K, int N,
                         const ProjWs &p, float *y, int *ks_out, const float **src_out, hipStream_t s)
 {
-    return gemm_ks ? enqueue_proj_gemm(ctx, prof, st_prod, W, rows, K, N, gemm_ks, p, y, ks_out, src_out, s)
-                   : enqueue_proj_few(ctx, prof, st_prod, W, rows, K, N, p, y, ks_out, src_out, s);
+    return p.route.gemm_ks ? enqueue_proj_gemm(ctx, prof, st_prod, W, rows, K, N, p, y, ks_out, src_out, s)
+                           : enqueue_proj_few(ctx, prof, st_prod, W, rows, K, N, p, y, ks_out, src_out, s);
 }
 
 int enqueue_proj(dmoe_ctx *ctx, bool prof, int st_conv, int st_prod, const WTensor &W, int rows, int K,
@@ -1569,9 +1470,9 @@ int enqueue_proj(dmoe_ctx *ctx, bool prof, int st_conv, int st_prod, const WTens
         STAGE(st_prod, launch_down_shared(W, x, N, K, rows, y, s));
         return DMOE_OK;
     }
-    if (proj_few(ctx->sw, path, rows, K, proj_chunk(ctx->sw, path, rows, K, N))) {
+    if (p.route.few) {
         // every token at once, or (Q6_K) chunks of up to PROJ_MAX_TOKENS
-        const int nc = proj_chunk(ctx->sw, path, rows, K, N);
+        const int nc = p.route.chunk;
         for (int t0 = 0; t0 < N; t0 += nc) {
             const int n = std::min(nc, N - t0);
             PrepJob pj{x + (size_t)t0 * K, n, K, ACT_SPLIT, p.act};
@@ -1581,12 +1482,12 @@ int enqueue_proj(dmoe_ctx *ctx, bool prof, int st_conv, int st_prod, const WTens
         }
         return DMOE_OK;
     }
-    if (const int ks = proj_gemm_slices(ctx->sw, path, rows, K, N)) {
-        // many tokens of Q4_K or Q6_K: the grouped GEMM's down launch over shared
+    if (p.route.gemm_ks) {
+        // many tokens of Q4_K or Q6_K, Q8_0: the grouped GEMM's down launch over shared
         // units, its reduction slices added in order
         PrepJob pj{x, N, K, path == DP_Q80 ? ACT_SPLIT32 : ACT_SPLIT, p.act};
         STAGE(st_conv, launch_prep(&pj, 1, s));
-        return enqueue_proj_gemm(ctx, prof, st_prod, W, rows, K, N, ks, p, y, nullptr, nullptr, s);
+        return enqueue_proj_gemm(ctx, prof, st_prod, W, rows, K, N, p, y, nullptr, nullptr, s);
     }
     LAUNCH_TRY(ctx, launch_fill_i32(p.n_ec, 0, 1, s));
     WorkList wl{};
@@ -1608,7 +1509,9 @@ int enqueue_proj(dmoe_ctx *ctx, bool prof, int st_conv, int st_prod, const WTens
         STAGE(st_prod, launch_gemm_f16(1, job, s));
         return DMOE_OK;
     }
+    // Q4_K and Q8_0 from here on (Q6_K has no item kernel: its route is never this one)
     const bool q8 = path == DP_Q80;
+    if (!q8 && path != DP_Q4K) return set_err(ctx, DMOE_ERR_UNSUPPORTED_TYPE, "projection: no kernel for type %d", W.type);
     if (!q8 && N <= DR_MAX_TOKENS && rows <= PROJ_ROWS_MAX) {
         // few tokens, up to a few thousand rows: one workgroup per 16 output
         // rows over every token (k_down_rows with the shared slot only), so
@@ -1737,8 +1640,8 @@ int enqueue_head(dmoe_ctx *ctx, const dmoe_layer *L, const HeadWs &w, const floa
     // :296-297 rms_norm(cur) * output_norm (h is only read: no residual add);
     // :299 the LM head.  On the few-token kernel or the GEMM the norm hands
     // the head its int8 digits directly.
-    int rc, gh = 0;
-    if (proj_takes_digits(ctx->sw, head_path(L->sd.type, V, H), V, H, N, &gh) && H <= 8192) {
+    int rc;
+    if (proj_takes_digits(w.proj, N) && H <= 8192) {
         NormArgs na{};
         na.h_in = h;
         na.gain = L->gate_w;
@@ -1747,7 +1650,7 @@ int enqueue_head(dmoe_ctx *ctx, const dmoe_layer *L, const HeadWs &w, const floa
         na.H = H;
         na.eps = eps;
         STAGE(ST_FRONT, launch_norm_fused(na, s));
-        rc = enqueue_proj_digits(ctx, prof, ST_SH_DOWN, L->sd, V, H, N, gh, w.proj, logits, nullptr, nullptr, s);
+        rc = enqueue_proj_digits(ctx, prof, ST_SH_DOWN, L->sd, V, H, N, w.proj, logits, nullptr, nullptr, s);
     } else {
         STAGE(ST_FRONT, launch_residual_rmsnorm(const_cast<float *>(h), nullptr, L->gate_w, w.xn, N, H, eps, s));
         rc = enqueue_proj(ctx, prof, ST_ACTQ_H, ST_SH_DOWN, L->sd, V, H, w.xn, N, logits, w.proj, s);
@@ -1807,12 +1710,11 @@ int enqueue_attn(dmoe_ctx *ctx, const dmoe_layer *L, const AttnWs &w, const floa
     const dmoe_attn_hparams &a = L->ahp;
     const int H = a.n_embd, QD = a.n_head * a.head_dim, KD = a.n_head_kv * a.head_dim, QKV = QD + 2 * KD;
     const bool prof = ctx->prof;
-    // Q4_K / Q6_K projections on the few-token kernel or the GEMM: the norms
+    // projections on the few-token kernel or the GEMM: the norms
     // hand them int8 digits and take their reduction slices directly
     // (k_norm_fused, k_qk_rope)
-    int gq = 0, go = 0;
-    const bool fq = proj_takes_digits(ctx->sw, head_path(L->aqkv.type, QKV, H), QKV, H, N, &gq) && H <= 8192;
-    const bool fo = proj_takes_digits(ctx->sw, head_path(L->awo.type, H, QD), H, QD, N, &go) && H <= 8192;
+    const bool fq = proj_takes_digits(w.pq, N) && H <= 8192;
+    const bool fo = proj_takes_digits(w.po, N) && H <= 8192;
 #define STAGE(id, call) LAUNCH_TRY(ctx, stage(ctx, prof, id, s, [&] { return call; }))
     // :120-121 input layernorm; :124 fused QKV
     const float *qkv = w.qkv;
@@ -1827,7 +1729,7 @@ int enqueue_attn(dmoe_ctx *ctx, const dmoe_layer *L, const AttnWs &w, const floa
         na.H = H;
         na.eps = a.rms_eps;
         STAGE(ST_FRONT, launch_norm_fused(na, s));
-        if ((rc = enqueue_proj_digits(ctx, prof, ST_SH_GATEUP, L->aqkv, QKV, H, N, gq, w.pq, w.qkv, &qks, &qkv, s)))
+        if ((rc = enqueue_proj_digits(ctx, prof, ST_SH_GATEUP, L->aqkv, QKV, H, N, w.pq, w.qkv, &qks, &qkv, s)))
             return rc;
     } else {
         STAGE(ST_FRONT, launch_residual_rmsnorm(const_cast<float *>(h), nullptr, L->attn_norm, w.xn, N, H,
@@ -1857,7 +1759,7 @@ int enqueue_attn(dmoe_ctx *ctx, const dmoe_layer *L, const AttnWs &w, const floa
         STAGE(ST_ACTQ_H, launch_prep(&pj, 1, s));
         const float *o = w.proj;
         int oks = 1;
-        if ((rc = enqueue_proj_digits(ctx, prof, ST_SH_DOWN, L->awo, H, QD, N, go, w.po, w.proj, &oks, &o, s)))
+        if ((rc = enqueue_proj_digits(ctx, prof, ST_SH_DOWN, L->awo, H, QD, N, w.po, w.proj, &oks, &o, s)))
             return rc;
         NormArgs na{};
         na.h_in = h;

@@ -7,6 +7,7 @@
 #include <stddef.h>
 
 #include "../../include/dmoe.h"
+#include "dmoe_plan.h"
 
 // Q8_K is an activation-only type (ggml id 15): the vec_dot_type of Q4_K.
 #define DMOE_ACT_Q8_K 15
@@ -123,25 +124,6 @@ struct MoeJob {
     // expert's as hi / lo pairs (lo rows after the hi rows)
     const uint16_t *x16, *xs16;
     uint16_t *h16, *hs16;
-};
-
-// Alternative kernels kept selectable for measurement, read from the
-// environment by dmoe_create into its context (never in a forward):
-//   DMOE_Q4K_COLUMN_BLOCKS = 1, 2, 4  column blocks of the Q4_K items (0: by tokens per expert)
-//   DMOE_DOWN_FUSED = 1               few-token Q4_K down products as the single fused launch
-//   DMOE_GATEUP_LDS = 1               the LDS-ring gate/up kernel instead of the register ring
-//   DMOE_EXPERT_TILE = 0 / 1          the tile kernels (k_expert_tile.hip) off / on for every N
-//   DMOE_EXPERT_GEMM = 0 / 1          the Q4_K grouped GEMM (k_expert_gemm.hip) off / on for every N
-//   DMOE_PROJ_GEMM = 0 / 1            Q4_K, Q6_K and Q8_0 projections (attention, LM head; Q4_K and Q6_K dense MLP)
-//                                     past the few-token kernels on that GEMM off / on for every N
-struct KernelSwitches {
-    int q4k_column_blocks = 0;
-    int expert_tile = -1;                // -1: by tokens per expert
-    int expert_gemm = -1;                // -1: by tokens per expert
-    int proj_gemm = -1;                  // -1: by tokens
-    int attn_waves = 0;                  // 0: by grid size, else 4 or 8 per workgroup
-    bool down_fused = false;
-    bool gateup_lds = false;
 };
 
 struct RouteParams {
@@ -265,7 +247,6 @@ hipError_t launch_argmax_prob(const float *logits, int N, int V, ArgmaxPart *par
 // Q4_K projections of few tokens with F32 weight semantics (k_proj.hip):
 // matrices w[0..M-1] (tiled Q4_K, R rows, reduction K) against x as two int8
 // digit rows per token (ACT_SPLIT); the reduction runs in KS slices.
-constexpr int PROJ_MAX_TOKENS = 32;
 struct ProjJob {
     const uint8_t *w[2];
     int32_t M, R, K, N, KS;
@@ -273,7 +254,6 @@ struct ProjJob {
     float *out;              // partial: [M][KS][N][R] slice sums; else y [N][ldo] (M = KS = 1)
     int32_t partial, ldo;
 };
-bool proj_ok(int R, int K, int N);
 struct ProjPlan {
     int T;                   // 16-row tiles per wavefront
     int KS;                  // reduction slices
@@ -310,7 +290,6 @@ hipError_t launch_expert_tile(int phase, const MoeJob &job, hipStream_t s);
 // / ys as with the tile kernels.  Without routed weights (a projection, the
 // dense MLP) also Q6_K, and Q8_0 for phase 1.
 constexpr int EXPERT_GEMM_CHUNK = 128;
-bool expert_gemm_q4k_ok(int H, int FF, int SF, bool shared);
 hipError_t launch_expert_gemm_q4k(int phase, const MoeJob &job, hipStream_t s);
 // Down products of the Q4_K experts and the weighted combine in one launch
 // for few tokens (k_down_rows.hip): one workgroup per 16 output rows, every

@@ -1,0 +1,148 @@
+// dmoe_plan.h — which kernels a projection, an LM head or a dense MLP takes:
+// pure host functions of the sizes, the weights' type and the context's
+// switches.  A call decides once, from all of its tokens, and plans its
+// workspace and launches its kernels from that one decision.  No HIP here:
+// tests/test_plan.py compiles this file for the CPU.
+#pragma once
+
+#include <stddef.h>
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace dmoe {
+
+// Alternative kernels kept selectable for measurement, read from the
+// environment by dmoe_create into its context (never in a forward):
+//   DMOE_Q4K_COLUMN_BLOCKS = 1, 2, 4  column blocks of the Q4_K items (0: by tokens per expert)
+//   DMOE_DOWN_FUSED = 1               few-token Q4_K down products as the single fused launch
+//   DMOE_GATEUP_LDS = 1               the LDS-ring gate/up kernel instead of the register ring
+//   DMOE_EXPERT_TILE = 0 / 1          the tile kernels (k_expert_tile.hip) off / on for every N
+//   DMOE_EXPERT_GEMM = 0 / 1          the Q4_K grouped GEMM (k_expert_gemm.hip) off / on for every N
+//   DMOE_PROJ_GEMM = 0 / 1            Q4_K, Q6_K and Q8_0 projections (attention, LM head; Q4_K and Q6_K dense MLP)
+//                                     past the few-token kernels on that GEMM off / on for every N
+struct KernelSwitches {
+    int q4k_column_blocks = 0;
+    int expert_tile = -1;                // -1: by tokens per expert
+    int expert_gemm = -1;                // -1: by tokens per expert
+    int proj_gemm = -1;                  // -1: by tokens
+    int attn_waves = 0;                  // 0: by grid size, else 4 or 8 per workgroup
+    bool down_fused = false;
+    bool gateup_lds = false;
+};
+
+// Kernel family of a matrix, by its type and shape (dense_path, head_path).
+enum WeightPath { DP_GEMV = 0, DP_Q4K, DP_Q80, DP_F16, DP_Q6K };
+
+// The few-token kernel (k_proj.hip): Q4_K and Q6_K, up to 32 tokens a launch.
+constexpr int PROJ_MAX_TOKENS = 32;
+
+inline bool proj_ok(int R, int K, int N)
+{
+    return R > 0 && R % 16 == 0 && K > 0 && K % 256 == 0 && N > 0 && N <= PROJ_MAX_TOKENS;
+}
+
+// Output rows up to which a few-token Q4_K projection runs one workgroup per
+// 16 rows (k_down_rows); above it (the LM head) the expert kernel's items.
+constexpr int PROJ_ROWS_MAX = 32768;
+
+// The grouped GEMM (k_expert_gemm.hip): rows of a gate/up and of a down item.
+constexpr int EXPERT_GEMM_GU_ROWS = 128, EXPERT_GEMM_DN_ROWS = 256;
+
+inline bool expert_gemm_q4k_ok(int H, int FF, int SF, bool shared)
+{
+    if (H % EXPERT_GEMM_DN_ROWS || FF % EXPERT_GEMM_GU_ROWS || H < 512 || FF < 512 || H % 256 || FF % 256) return false;
+    if (shared && SF != FF) return false;
+    return true;
+}
+
+// Q4_K, Q6_K and Q8_0 projections of proj_gemm_min_tokens or more tokens run on the
+// grouped GEMM's down launch (k_expert_gemm.hip) with shared units only: 64 tokens
+// (128 digit rows) per unit, 256 output rows per item, the reduction split
+// into slices of 2 or more super-blocks, as many as minimise the static
+// schedule's rounds x steps plus the slices' own traffic.  Returns the slice
+// count, 0 where the GEMM does not take the shape.
+constexpr int PROJ_GEMM_MIN_TOKENS = 33;
+
+// Q6_K matrices of an LM head's rows take the GEMM (in units of 32 tokens)
+// from 17 tokens on: at 157,184 x 4,096 rows 16 / 17 / 24 / 32 tokens 145 / 167
+// / 172 / 177 us against 140 / 174 / 177 / 217 on the few-token kernel, whose
+// work per weight grows by the eight tokens.  A few thousand rows fill too few
+// of the GEMM's 256-row items.
+constexpr int PROJ_GEMM_MIN_TOKENS_Q6K_HEAD = 17;
+
+// Q8_0 projections have no few-token kernel of their own: against the expert
+// kernel's items of 8 tokens the GEMM takes the attention half of 1 / 8 / 20
+// tokens from 95 / 98 / 99 us to 46 / 49 / 53, and an LM head of 16 / 32 tokens
+// from 233 / 468 us to 160 / 194; one item of the expert kernel covers a head
+// of up to 8 tokens (128 / 133 us at 1 / 8 tokens against 137 / 148).
+constexpr int PROJ_GEMM_MIN_TOKENS_Q80 = 1, PROJ_GEMM_MIN_TOKENS_Q80_HEAD = 9;
+
+inline int proj_gemm_min_tokens(int path, int rows)
+{
+    if (path == DP_Q80) return rows > PROJ_ROWS_MAX ? PROJ_GEMM_MIN_TOKENS_Q80_HEAD : PROJ_GEMM_MIN_TOKENS_Q80;
+    return path == DP_Q6K && rows > PROJ_ROWS_MAX ? PROJ_GEMM_MIN_TOKENS_Q6K_HEAD : PROJ_GEMM_MIN_TOKENS;
+}
+
+inline int proj_gemm_slices(const KernelSwitches &sw, int path, int rows, int K, int N, int n_cu)
+{
+    if ((path != DP_Q4K && path != DP_Q6K && path != DP_Q80) || sw.proj_gemm == 0 ||
+        (sw.proj_gemm < 0 && N < proj_gemm_min_tokens(path, rows)) ||
+        !expert_gemm_q4k_ok(rows, K, K, true) || 2L * N * K >= (1L << 31))
+        return 0;
+    const long items = (long)((N + 63) / 64) * (rows / 256);
+    const int nsb = K / 256;
+    const long grid = (n_cu + 7) / 8 * 8;
+    // rounds of the static schedule x super-blocks per item at ~4.5 us per
+    // step, plus the slices written and read again at ~4 TB/s
+    int best = 1;
+    double best_us = 0.0;
+    for (int ks = 1; ks <= 16; ks *= 2) {
+        if (nsb % ks || (ks > 1 && nsb / ks < 2)) continue;
+        const long rounds = (items * ks + grid - 1) / grid;
+        double us = 4.5 * (double)(rounds * (nsb / ks));
+        if (ks > 1) us += (double)ks * N * rows * 8 / 4e6;
+        if (ks == 1 || us < best_us) {
+            best = ks;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
+// What a projection y [N][rows] = W x, or a dense MLP, runs on:
+//   few          the few-token kernel, `chunk` tokens a launch (Q6_K of any N:
+//                it has no item kernel; Q4_K in one launch)
+//   gemm_ks > 0  the grouped GEMM over all tokens, the (down) reduction in
+//                gemm_ks slices
+//   neither      the item kernels over all tokens
+// `chunk` is the tokens whose converted activations are held at once.
+struct ProjRoute {
+    bool few;
+    int gemm_ks;
+    int chunk;
+};
+
+inline ProjRoute proj_route(const KernelSwitches &sw, int path, int rows, int K, int N, int n_cu)
+{
+    ProjRoute r{false, proj_gemm_slices(sw, path, rows, K, N, n_cu), N};
+    const bool int4_6 = path == DP_Q4K || path == DP_Q6K;
+    if (int4_6 && proj_ok(rows, K, N) && (N < proj_gemm_min_tokens(path, rows) || !r.gemm_ks))
+        return ProjRoute{true, 0, N};
+    if (path == DP_Q6K && !r.gemm_ks) return ProjRoute{true, 0, std::min(N, PROJ_MAX_TOKENS)};
+    return r;
+}
+
+// The dense MLP: gate and up as one two-matrix projection and down as
+// another, both on the few-token kernel (Q6_K past it in chunks, where the
+// GEMM does not take the shape), or the GEMM's gate/up and down launches.
+inline ProjRoute dense_route(const KernelSwitches &sw, int path, int H, int FF, int N, int n_cu)
+{
+    const int ks = path == DP_Q80 || 2L * N * H >= (1L << 31) ? 0 : proj_gemm_slices(sw, path, H, FF, N, n_cu);
+    const int chunk = path == DP_Q6K && !ks ? std::min(N, PROJ_MAX_TOKENS) : N;
+    const bool int4_6 = path == DP_Q4K || path == DP_Q6K;
+    if (int4_6 && proj_ok(FF, H, chunk) && proj_ok(H, FF, chunk)) return ProjRoute{true, 0, chunk};
+    return ProjRoute{false, ks, N};
+}
+
+} // namespace dmoe

@@ -342,7 +342,8 @@ hipError_t launch_down_rows(const DownRowsJob &job, hipStream_t s)
     if (!down_rows_ok(job.N, job.K, job.E, job.H, job.FF) ||
         job.ec_cap + (job.has_shared ? (job.N + 7) / 8 : 0) > DR_MAX_UNITS ||
         job.wl.chunk != EXPERT_CHUNK || (job.K > 0 && job.ah.K != job.FF) ||
-        (job.has_shared && job.ahs.K != job.FF) || (job.K == 0 && (!job.has_shared || job.ec_cap != 0)))
+        (job.has_shared && job.ahs.K != job.FF) || (job.K == 0 && (!job.has_shared || job.ec_cap != 0)) ||
+        (job.ed.data && job.ed.type != DMOE_TYPE_Q4_K) || (job.sd.data && job.sd.type != DMOE_TYPE_Q4_K))
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_down_rows, dim3(job.H / 16), dim3(DR_WAVES * 64), 0, s, job);
     return hipGetLastError();

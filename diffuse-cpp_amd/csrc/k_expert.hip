@@ -737,6 +737,8 @@ hipError_t launch_expert_q4k(int phase, const MoeJob &job, hipStream_t s, int nc
         job.ax.K != job.H || job.ah.K != job.FF ||
         (job.has_shared && (job.SF != job.FF || job.ahs.K != job.SF)))
         return hipErrorInvalidValue;
+    for (const WTensor *w : {&job.eg, &job.eu, &job.ed, &job.sg, &job.su, &job.sd})
+        if (w->data && w->type != DMOE_TYPE_Q4_K) return hipErrorInvalidValue;
     // routed work-list entries hold 16 nc pairs
     if ((nc != 1 && nc != 2 && nc != 4) || (job.wl.n_ec && job.wl.chunk != EXPERT_CHUNK * nc))
         return hipErrorInvalidValue;

@@ -90,6 +90,7 @@ constexpr int XG_AD = XG_ABS + 1024;                         // scales: [32] f32
 constexpr int XG_ABLK = XG_AD + 128;                         // one block (9,344)
 constexpr int XG_AHEAD = 4;                                  // operand reads ahead of their MFMAs (divides 8)
 static_assert(XG_ABLK % 16 == 0, "16-byte pieces");
+static_assert(XG_GU_ROWS == EXPERT_GEMM_GU_ROWS && XG_DN_ROWS == EXPERT_GEMM_DN_ROWS, "the dispatch's item rows");
 
 // Item k is row group k % rg_n of unit k / rg_n; a unit is shared chunk
 // u < nch, else work-list entry u - nch.  Every field is wave-uniform.
@@ -908,13 +909,6 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
 }
 
 // ---------------------------------------------------------------------------
-bool expert_gemm_q4k_ok(int H, int FF, int SF, bool shared)
-{
-    if (H % XG_DN_ROWS || FF % XG_GU_ROWS || H < 512 || FF < 512 || H % 256 || FF % 256) return false;
-    if (shared && SF != FF) return false;
-    return true;
-}
-
 // One workgroup per CU (the two stages fill the LDS), a multiple of 8 (one
 // row group per XCD); each runs its items until the schedule's units end.
 hipError_t launch_expert_gemm_q4k(int phase, const MoeJob &job, hipStream_t s)

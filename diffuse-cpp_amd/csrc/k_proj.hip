@@ -614,11 +614,6 @@ ProjPlan proj_plan(int R, int K, int M, int N)
     return best;
 }
 
-bool proj_ok(int R, int K, int N)
-{
-    return R > 0 && R % 16 == 0 && K > 0 && K % 256 == 0 && N > 0 && N <= PROJ_MAX_TOKENS;
-}
-
 size_t proj_partial_floats(int R, int K, int M, int N)
 {
     return (size_t)M * proj_plan(R, K, M, N).KS * N * R;

@@ -1,0 +1,81 @@
+"""CPU: the choice of kernels for projections, LM heads and dense MLPs
+(csrc/dmoe_plan.h, pure host functions) over every type, the corners of each
+kernel's range and the sizes around the 32-bit limits: the workspace is
+planned for the tokens that the chosen kernel converts, and the chosen kernel
+takes the type and the shape."""
+import itertools
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+GEMV, Q4K, Q80, F16, Q6K = range(5)
+N_CU = 256
+
+PROBE = r"""
+#include <cstdio>
+#include "%s"
+using namespace dmoe;
+int main() {
+  char kind; int path, rows, K, N, force;
+  while (scanf(" %%c %%d %%d %%d %%d %%d", &kind, &path, &rows, &K, &N, &force) == 6) {
+    KernelSwitches sw;
+    sw.proj_gemm = force;
+    const ProjRoute r = kind == 'p' ? proj_route(sw, path, rows, K, N, 256) : dense_route(sw, path, rows, K, N, 256);
+    printf("%%d %%d %%d\n", r.few, r.gemm_ks, r.chunk);
+  }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def routes(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plan")
+    src = d / "probe.cpp"
+    src.write_text(PROBE % (ROOT / "diffuse-cpp_amd" / "csrc" / "dmoe_plan.h"))
+    subprocess.run(["g++", "-std=c++17", "-O1", "-o", str(d / "probe"), str(src)], check=True)
+
+    def ask(cases):
+        """[(kind, path, rows, K, N, DMOE_PROJ_GEMM or -1)] -> [(few, gemm_ks, chunk)];
+        a dense MLP's rows and K are its n_embd and n_ff"""
+        text = "\n".join(" ".join(map(str, c)) for c in cases)
+        out = subprocess.run([str(d / "probe")], input=text, capture_output=True, text=True, check=True).stdout
+        got = [tuple(map(int, line.split())) for line in out.splitlines()]
+        assert len(got) == len(cases)
+        return got
+    return ask
+
+
+def _fits(kind, path, rows, K, N, few, ks, chunk):
+    """The kernel of the route takes the call, in the chunk that is planned."""
+    if few:
+        # converted activations: one chunk, reused; only Q6_K runs in several
+        ok = path in (Q4K, Q6K) and 0 < chunk <= 32 and rows % 16 == 0 and K % 256 == 0 and ks == 0
+        return ok and (chunk == N or path == Q6K)
+    if ks:
+        # 32-bit offsets into the converted activations (two digit rows a token)
+        widest = max(rows, K) if kind == "d" else K
+        steps = K // 256 // ks
+        return (path in (Q4K, Q6K, Q80) and chunk == N and 2 * N * widest < 2 ** 31 and rows % 256 == 0
+                and K % 256 == 0 and K // 256 % ks == 0 and (steps >= 2))
+    return path in (Q4K, Q80) and chunk == N        # the item kernels
+
+
+def test_a_route_fits_what_is_planned(routes):
+    rows = [16, 256, 272, 512, 1024, 32768, 33024, 33040, 157184]
+    ks = [256, 512, 2816, 4096, 8192, 16640]
+    ns = [1, 8, 9, 16, 17, 24, 25, 32, 33, 64, 65, 2048, 64528, 64529, 131071, 131072, 262143, 262144, 300000]
+    cases = [("p",) + c for c in itertools.product((Q4K, Q6K, Q80), rows, ks, ns, (-1, 0, 1))]
+    cases += [("d",) + c for c in itertools.product((Q4K, Q6K, Q80), (256, 512, 4096, 16640), ks, ns, (-1, 0, 1))]
+    for c, r in zip(cases, routes(cases)):
+        kind, path, R, K, N, _ = c
+        assert _fits(kind, path, R, K, N, *r), (c, r)
+
+
+@pytest.mark.parametrize("N,K", [(262144, 4096), (131072, 8192), (64529, 16640)])
+def test_q6k_head_past_the_gemm_runs_in_chunks(routes, N, K):
+    """A Q6_K head of more tokens than the GEMM's 32-bit offsets reach: chunks
+    of the few-token kernel, although the GEMM takes such a chunk by itself."""
+    assert routes([("p", Q6K, 157184, K, N, -1)]) == [(1, 0, 32)]
+    assert routes([("p", Q6K, 157184, K, 2 ** 31 // (2 * K) - 1, -1)])[0][1] > 0
