@@ -1202,8 +1202,9 @@ int ensure_dense_workspace(dmoe_ctx *ctx, const dmoe_layer *L, int N, bool host_
     return DMOE_OK;
 }
 
-int enqueue_dense(dmoe_ctx *ctx, const dmoe_layer *L, const DenseWs &w, const float *x, int N,
-                  float *y, hipStream_t s, bool prof)
+// sw: the switches that w was planned with
+int enqueue_dense(dmoe_ctx *ctx, const KernelSwitches &sw, const dmoe_layer *L, const DenseWs &w, const float *x,
+                  int N, float *y, hipStream_t s, bool prof)
 {
     const int H = L->hp.n_embd, FF = L->hp.shared_ff;
     const int path = dense_path(L->sg.type, H, FF);
@@ -1213,7 +1214,7 @@ int enqueue_dense(dmoe_ctx *ctx, const dmoe_layer *L, const DenseWs &w, const fl
         STAGE(ST_SH_DOWN, launch_down_shared(L->sd, w.hs, N, FF, H, y, s));
         return DMOE_OK;
     }
-    const ProjRoute r = dense_route(ctx->sw, path, H, FF, N, plan_cus());
+    const ProjRoute r = dense_route(sw, path, H, FF, N, plan_cus());
     if (r.few) {
         // gate and up: one launch over both matrices, h from their slices;
         // tokens t0 .. t0 + n - 1 at a time (every token at once, or Q6_K chunks)
@@ -1330,7 +1331,7 @@ int enqueue_dense(dmoe_ctx *ctx, const dmoe_layer *L, const DenseWs &w, const fl
     job.ys = y;                          // the shared expert's down output is the MLP's
     PrepJob pj{x, N, H, q8 ? ACT_SPLIT32 : ACT_SPLIT, w.axs};
     STAGE(ST_ACTQ_X, launch_prep(&pj, 1, s));
-    STAGE(ST_SH_GATEUP, q8 ? launch_expert_q80(0, job, s) : launch_expert_q4k(0, job, s, 1, ctx->sw.gateup_lds));
+    STAGE(ST_SH_GATEUP, q8 ? launch_expert_q80(0, job, s) : launch_expert_q4k(0, job, s, 1, sw.gateup_lds));
     STAGE(ST_SH_DOWN, q8 ? launch_expert_q80(1, job, s) : launch_expert_q4k(1, job, s));
 #undef STAGE
     return DMOE_OK;
@@ -2268,7 +2269,7 @@ int dmoe_layer_forward(dmoe_ctx *ctx, const dmoe_layer *L, const float *x, int32
         if (rc) return rc;
         hipStream_t s = ctx->stream;
         HIP_TRY(ctx, hipMemcpyAsync(dw.x, x, (size_t)n_tokens * H * 4, hipMemcpyHostToDevice, s));
-        if ((rc = enqueue_dense(ctx, L, dw, dw.x, n_tokens, dw.y, s, ctx->prof))) return rc;
+        if ((rc = enqueue_dense(ctx, ctx->sw, L, dw, dw.x, n_tokens, dw.y, s, ctx->prof))) return rc;
         HIP_TRY(ctx, hipMemcpyAsync(y, dw.y, (size_t)n_tokens * H * 4, hipMemcpyDeviceToHost, s));
         if (dbg && dbg->use_block_routing) *dbg->use_block_routing = 0;
         HIP_TRY(ctx, hipStreamSynchronize(s));
@@ -2301,7 +2302,7 @@ int dmoe_layer_forward_device(dmoe_ctx *ctx, const dmoe_layer *L, const float *x
         DenseWs dw;
         int rc = ensure_dense_workspace(ctx, L, n_tokens, false, &dw);
         if (rc) return rc;
-        return enqueue_dense(ctx, L, dw, x_dev, n_tokens, y_dev, (hipStream_t)stream, ctx->prof);
+        return enqueue_dense(ctx, ctx->sw, L, dw, x_dev, n_tokens, y_dev, (hipStream_t)stream, ctx->prof);
     }
     Workspace w;
     int rc = ensure_workspace(ctx, L, n_tokens, false, &w);
@@ -2324,9 +2325,18 @@ int dmoe_layer_forward_device_noalloc(dmoe_ctx *ctx, const dmoe_layer *L, const 
                        L->device, ctx->device);
     if (!ctx->scratch)
         return set_err(ctx, DMOE_ERR_HIP, "scratch address of device %d not resolved", ctx->device);
-    const size_t need = L->dense ? plan_dense(ctx->sw, L, n_tokens, false, nullptr, nullptr)
-                                 : plan_workspace(ctx->sw, L->hp, L->eg.type, L->sg.type, L->has_shared, n_tokens,
-                                                  false, nullptr, nullptr);
+    KernelSwitches sw = ctx->sw;
+    size_t need = L->dense ? plan_dense(sw, L, n_tokens, false, nullptr, nullptr)
+                           : plan_workspace(sw, L->hp, L->eg.type, L->sg.type, L->has_shared, n_tokens,
+                                            false, nullptr, nullptr);
+    if (L->dense && need > DMOE_NOALLOC_SCRATCH_BYTES &&
+        dense_path(L->sg.type, L->hp.n_embd, L->hp.shared_ff) == DP_Q6K) {
+        // a Q6_K MLP whose GEMM workspace (every token's activations and h)
+        // does not fit runs in the few-token kernel's chunks, which need room
+        // for 32 tokens at any count
+        sw.proj_gemm = 0;
+        need = plan_dense(sw, L, n_tokens, false, nullptr, nullptr);
+    }
     if (need > DMOE_NOALLOC_SCRATCH_BYTES)
         return set_err(ctx, DMOE_ERR_INVALID_ARG,
                        "n_tokens = %d needs %zu bytes of workspace, above the %zu-byte scratch of "
@@ -2337,8 +2347,8 @@ int dmoe_layer_forward_device_noalloc(dmoe_ctx *ctx, const dmoe_layer *L, const 
     // what a previous call left in the scratch needs no clearing.
     if (L->dense) {
         DenseWs dw;
-        plan_dense(ctx->sw, L, n_tokens, false, ctx->scratch, &dw);
-        return enqueue_dense(ctx, L, dw, x_dev, n_tokens, y_dev, (hipStream_t)stream, false);
+        plan_dense(sw, L, n_tokens, false, ctx->scratch, &dw);
+        return enqueue_dense(ctx, sw, L, dw, x_dev, n_tokens, y_dev, (hipStream_t)stream, false);
     }
     Workspace w;
     plan_workspace(ctx->sw, L->hp, L->eg.type, L->sg.type, L->has_shared, n_tokens, false, ctx->scratch, &w);
