@@ -355,12 +355,17 @@ bool use_gemm_path(const dmoe_hparams &hp, int32_t wtype, int32_t stype, bool sh
 // grouped GEMM of 256-pair items).  DMOE_EXPERT_TILE = 0 / 1 turns the
 // choice off / on for every N (with the shapes the tile kernels take).
 // The Q4_K grouped GEMM of k_expert_gemm.hip (units of up to 128 pairs, each
-// step's weight tiles applied to all of a unit's pairs): by the forward's
-// pairs per expert averaged over all experts, N k / E of at least
-// GEMM_Q4K_MIN_AVG (the flash layer: 1,024 tokens 597 us against 635 on the tile kernels, 512
-// tokens 394 against 386, 256 tokens 284 against 264).  DMOE_EXPERT_GEMM = 0 / 1 turns it off / on for every N;
-// DMOE_EXPERT_TILE or DMOE_Q4K_COLUMN_BLOCKS set selects their kernels.
-constexpr long GEMM_Q4K_MIN_AVG = 32;
+// step's weight tiles applied to all of a unit's pairs): by moe_gemm_pays.
+// DMOE_EXPERT_GEMM = 0 / 1 turns it off / on for every N; DMOE_EXPERT_TILE or
+// DMOE_Q4K_COLUMN_BLOCKS set selects their kernels.
+bool block_routed(const dmoe_hparams &hp, int N);
+
+// The compute units the routes are planned for (without a device: a whole chip).
+int plan_cus()
+{
+    int n_cu = 0;
+    return device_cu_count(&n_cu) == hipSuccess ? n_cu : 256;
+}
 
 bool use_q4k_gemm(const KernelSwitches &sw, const dmoe_hparams &hp, int32_t wtype, int32_t stype, bool shared,
                   int N)
@@ -371,8 +376,8 @@ bool use_q4k_gemm(const KernelSwitches &sw, const dmoe_hparams &hp, int32_t wtyp
     if ((long)N * hp.top_k * hp.moe_ff >= (1L << 31) || 2L * N * hp.n_embd >= (1L << 31)) return false;
     if (sw.expert_gemm >= 0) return sw.expert_gemm == 1;
     if (sw.expert_tile >= 0 || sw.q4k_column_blocks) return false;
-    const long avg = (long)N * hp.top_k / (hp.n_experts > 0 ? hp.n_experts : 1);
-    return avg >= GEMM_Q4K_MIN_AVG;
+    return moe_gemm_pays(N, hp.top_k, hp.n_experts, hp.moe_ff, shared, block_routed(hp, N),
+                         expert_tile_ok(hp.n_embd, hp.moe_ff, hp.shared_ff, shared), plan_cus());
 }
 
 bool use_tile_path(const KernelSwitches &sw, const dmoe_hparams &hp, int32_t wtype, int32_t stype, bool shared,
@@ -584,6 +589,12 @@ int ensure_workspace(dmoe_ctx *ctx, const dmoe_layer *L, int N, bool host_io, Wo
     return DMOE_OK;
 }
 
+// src/diffuse-moe-graph.cpp:215-216
+bool block_routed(const dmoe_hparams &hp, int N)
+{
+    return hp.block_size > 1 && hp.capacity > 0 && hp.capacity < hp.n_experts && N % hp.block_size == 0;
+}
+
 RouteParams route_params(const dmoe_layer *L, const dmoe_hparams &hp, int N)
 {
     RouteParams rp{};
@@ -594,9 +605,7 @@ RouteParams route_params(const dmoe_layer *L, const dmoe_hparams &hp, int N)
     rp.top_k = hp.top_k;
     rp.capacity = hp.capacity;
     rp.block_size = hp.block_size;
-    // src/diffuse-moe-graph.cpp:215-216
-    rp.use_block = hp.block_size > 1 && hp.capacity > 0 && hp.capacity < hp.n_experts &&
-                   N % hp.block_size == 0;
+    rp.use_block = block_routed(hp, N);
     rp.norm_topk_prob = hp.norm_topk_prob;
     rp.routed_scaling = hp.routed_scaling;
     return rp;
@@ -1093,13 +1102,6 @@ struct DenseWs {
     float *hs;                           // f32 h (GEMV path)
     float *part_gu, *part_d;             // slice sums of the few-token Q4_K projections
 };
-
-// The compute units the routes are planned for (without a device: a whole chip).
-int plan_cus()
-{
-    int n_cu = 0;
-    return device_cu_count(&n_cu) == hipSuccess ? n_cu : 256;
-}
 
 // Slice-sum floats the few-token projection of R x K (M matrices) needs at
 // any token count 1 .. nmax (a smaller last chunk may split its reduction

@@ -1,5 +1,5 @@
-// dmoe_plan.h — which kernels a projection, an LM head or a dense MLP takes:
-// pure host functions of the sizes, the weights' type and the context's
+// dmoe_plan.h — which kernels a projection, an LM head, a dense MLP or a routed
+// layer's Q4_K experts take: pure host functions of the sizes, the weights' type and the context's
 // switches.  A call decides once, from all of its tokens, and plans its
 // workspace and launches its kernels from that one decision.  No HIP here:
 // tests/test_plan.py compiles this file for the CPU.
@@ -54,6 +54,32 @@ inline bool expert_gemm_q4k_ok(int H, int FF, int SF, bool shared)
     if (H % EXPERT_GEMM_DN_ROWS || FF % EXPERT_GEMM_GU_ROWS || H < 512 || FF < 512 || H % 256 || FF % 256) return false;
     if (shared && SF != FF) return false;
     return true;
+}
+
+// Whether the routed Q4_K experts of N tokens take the GEMM (units of up to 128
+// pairs) rather than the tile kernels (units of up to 32).  From 64 pairs per
+// expert on, averaged over all experts, always.  From 32 on it depends on
+// whether its larger items still fill the chip and whether the pairs fill its
+// blocks of 32: block routing gathers a block's pairs on few experts, plain
+// top-k leaves each with about the average.  Items below are the gate/up
+// launch's, one unit per expert.  Measured (tile kernels against GEMM, us):
+//   4,096 x 1,024, 256 experts, top 8 (2,176 items): 1,024 tokens 666 / 591, 1,025 752 / 727
+//   2,048 x 512, 256 experts, top 8 (1,088): 1,024 tokens 245 / 233, 1,025 280 / 282, 1,409 322 / 314
+//   2,048 x 512, 128 experts, top 8 (544): 512 tokens 148 / 124, 513 158 / 167
+//   2,048 x 1,024, 16 experts, top 2 (160): 256 tokens 88 / 98; 480 92 / 101
+//   1,024 x 512, 32 experts, top 4 (144): 256 tokens 58 / 74; 480 70 / 77
+// Where the tile kernels do not take the shape (moe_ff 2,048), the GEMM is
+// ahead of the item kernels from 32 on: 4,096 x 2,048, 8 experts, top 2, 128
+// tokens 172 / 152.
+constexpr long GEMM_Q4K_MIN_AVG = 32, GEMM_Q4K_MIN_AVG_PLAIN = 40, GEMM_Q4K_ANY_AVG = 64;
+
+inline bool moe_gemm_pays(int N, int top_k, int E, int FF, bool shared, bool block_routing, bool tile_ok, int n_cu)
+{
+    const long avg = (long)N * top_k / (E > 0 ? E : 1);
+    if (avg >= GEMM_Q4K_ANY_AVG || avg < GEMM_Q4K_MIN_AVG) return avg >= GEMM_Q4K_ANY_AVG;
+    if (!tile_ok) return true;
+    const long items = (long)(E + (shared ? (N + 63) / 64 : 0)) * (FF / EXPERT_GEMM_GU_ROWS);
+    return block_routing ? items >= 2L * n_cu : avg >= GEMM_Q4K_MIN_AVG_PLAIN && items >= 3L * n_cu;
 }
 
 // Q4_K, Q6_K and Q8_0 projections of proj_gemm_min_tokens or more tokens run on the

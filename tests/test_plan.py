@@ -1,5 +1,5 @@
-"""CPU: the choice of kernels for projections, LM heads and dense MLPs
-(csrc/dmoe_plan.h, pure host functions) over every type, the corners of each
+"""CPU: the choice of kernels for projections, LM heads, dense MLPs and routed
+Q4_K experts (csrc/dmoe_plan.h, pure host functions) over every type, the corners of each
 kernel's range and the sizes around the 32-bit limits: the workspace is
 planned for the tokens that the chosen kernel converts, and the chosen kernel
 takes the type and the shape."""
@@ -22,6 +22,10 @@ int main() {
   while (scanf(" %%c %%d %%d %%d %%d %%d", &kind, &path, &rows, &K, &N, &force) == 6) {
     KernelSwitches sw;
     sw.proj_gemm = force;
+    if (kind == 'm') {      // a routed layer: top_k, experts, moe_ff, tokens, block routing (2: no tile kernels)
+      printf("%%d 0 0\n", moe_gemm_pays(N, path, rows, K, true, force & 1, force < 2, 256));
+      continue;
+    }
     const ProjRoute r = kind == 'p' ? proj_route(sw, path, rows, K, N, 256) : dense_route(sw, path, rows, K, N, 256);
     printf("%%d %%d %%d\n", r.few, r.gemm_ks, r.chunk);
   }
@@ -79,3 +83,15 @@ def test_q6k_head_past_the_gemm_runs_in_chunks(routes, N, K):
     of the few-token kernel, although the GEMM takes such a chunk by itself."""
     assert routes([("p", Q6K, 157184, K, N, -1)]) == [(1, 0, 32)]
     assert routes([("p", Q6K, 157184, K, 2 ** 31 // (2 * K) - 1, -1)])[0][1] > 0
+
+
+@pytest.mark.parametrize("top_k,E,FF,N,block,gemm", [
+    (8, 256, 1024, 1023, 0, 0), (8, 256, 1024, 1024, 1, 1), (8, 256, 1024, 1025, 0, 0), (8, 256, 1024, 1409, 0, 1),
+    (8, 256, 512, 992, 1, 0), (8, 256, 512, 1024, 1, 1), (8, 128, 512, 512, 1, 1), (8, 128, 512, 705, 0, 0),
+    (2, 16, 1024, 256, 1, 0), (2, 16, 1024, 480, 1, 0), (2, 16, 1024, 512, 1, 1), (4, 32, 512, 384, 1, 0),
+    (6, 64, 1024, 352, 1, 1), (6, 64, 1024, 342, 0, 0), (2, 8, 2048, 128, 2, 1), (2, 8, 2048, 112, 2, 0)])
+def test_routed_q4k_gemm(routes, top_k, E, FF, N, block, gemm):
+    """Between 32 and 64 pairs per expert the grouped GEMM only where it
+    measured ahead of the tile kernels: enough items, and with plain top-k
+    more pairs per expert."""
+    assert routes([("m", top_k, E, FF, N, block)])[0][0] == gemm
