@@ -86,8 +86,15 @@ inline bool moe_gemm_pays(int N, int top_k, int E, int FF, bool shared, bool blo
 // grouped GEMM's down launch (k_expert_gemm.hip) with shared units only: 64 tokens
 // (128 digit rows) per unit, 256 output rows per item, the reduction split
 // into slices of 2 or more super-blocks, as many as minimise the static
-// schedule's rounds x steps plus the slices' own traffic.  Returns the slice
-// count, 0 where the GEMM does not take the shape.
+// schedule's rounds x steps plus the slices' own traffic.  ks is the slice
+// count, 0 where the GEMM does not take the shape; rounds the workgroups' items
+// one after another, us the estimate.
+struct ProjGemm {
+    int ks;
+    long rounds;
+    double us;
+};
+
 constexpr int PROJ_GEMM_MIN_TOKENS = 33;
 
 // Q6_K matrices of an LM head's rows take the GEMM (in units of 32 tokens)
@@ -101,7 +108,8 @@ constexpr int PROJ_GEMM_MIN_TOKENS_Q6K_HEAD = 17;
 // kernel's items of 8 tokens the GEMM takes the attention half of 1 / 8 / 20
 // tokens from 95 / 98 / 99 us to 46 / 49 / 53, and an LM head of 16 / 32 tokens
 // from 233 / 468 us to 160 / 194; one item of the expert kernel covers a head
-// of up to 8 tokens (128 / 133 us at 1 / 8 tokens against 137 / 148).
+// of up to 8 tokens (128 / 133 us at 1 / 8 tokens against 137 / 148).  Between
+// these q80_gemm_pays weighs the two.
 constexpr int PROJ_GEMM_MIN_TOKENS_Q80 = 1, PROJ_GEMM_MIN_TOKENS_Q80_HEAD = 9;
 
 inline int proj_gemm_min_tokens(int path, int rows)
@@ -110,30 +118,45 @@ inline int proj_gemm_min_tokens(int path, int rows)
     return path == DP_Q6K && rows > PROJ_ROWS_MAX ? PROJ_GEMM_MIN_TOKENS_Q6K_HEAD : PROJ_GEMM_MIN_TOKENS;
 }
 
-inline int proj_gemm_slices(const KernelSwitches &sw, int path, int rows, int K, int N, int n_cu)
+inline ProjGemm proj_gemm(const KernelSwitches &sw, int path, int rows, int K, int N, int n_cu)
 {
+    ProjGemm g{0, 0, 0.0};
     if ((path != DP_Q4K && path != DP_Q6K && path != DP_Q80) || sw.proj_gemm == 0 ||
         (sw.proj_gemm < 0 && N < proj_gemm_min_tokens(path, rows)) ||
         !expert_gemm_q4k_ok(rows, K, K, true) || 2L * N * K >= (1L << 31))
-        return 0;
+        return g;
     const long items = (long)((N + 63) / 64) * (rows / 256);
     const int nsb = K / 256;
     const long grid = (n_cu + 7) / 8 * 8;
     // rounds of the static schedule x super-blocks per item at ~4.5 us per
     // step, plus the slices written and read again at ~4 TB/s
-    int best = 1;
-    double best_us = 0.0;
     for (int ks = 1; ks <= 16; ks *= 2) {
         if (nsb % ks || (ks > 1 && nsb / ks < 2)) continue;
         const long rounds = (items * ks + grid - 1) / grid;
         double us = 4.5 * (double)(rounds * (nsb / ks));
         if (ks > 1) us += (double)ks * N * rows * 8 / 4e6;
-        if (ks == 1 || us < best_us) {
-            best = ks;
-            best_us = us;
-        }
+        if (ks == 1 || us < g.us) g = ProjGemm{ks, rounds, us};
     }
-    return best;
+    return g;
+}
+
+// Q8_0: the GEMM g against the expert kernel's items of 8 tokens x 256 rows,
+// which spread few rows over more compute units and take an item's whole
+// reduction at about 2.2 us per super-block.  A step of the GEMM lasts 2 / 3 /
+// 4 / 5 us with up to 16 / 32 / 48 / 64 tokens in a unit; slices cost a few us
+// and their traffic, the item kernel a conversion launch (1 us).  A head of
+// 405 shapes (512 to 16,384 rows x 512 to 4,096, 1 to 512 tokens) measured on
+// both, items / GEMM: 2,048 x 512 at 16 tokens 22 / 20 us, at 64 22 / 27; 4,096 x
+// 1,024 at 32 tokens 26 / 25, at 48 26 / 27; 4,096 x 2,816 (a prime number of
+// super-blocks: one slice) at 16 tokens 39 / 36, at 32 39 / 46, at 128 41 / 71;
+// 16,384 x 2,816 at 64 tokens 63 / 72, at 96 86 / 72.
+inline bool q80_gemm_pays(const ProjGemm &g, int rows, int K, int N, int n_cu)
+{
+    const long grid = (n_cu + 7) / 8 * 8, items = (long)((N + 7) / 8) * (rows / 256);
+    const int nsb = K / 256;
+    double gemm_us = (1.0 + std::min(4, (N + 15) / 16)) * (double)(g.rounds * (nsb / g.ks));
+    if (g.ks > 1) gemm_us += 3.0 + (double)g.ks * N * rows * 8 / 4e6;
+    return gemm_us <= 2.2 * nsb * (double)((items + grid - 1) / grid) + 1.0;
 }
 
 // What a projection y [N][rows] = W x, or a dense MLP, runs on:
@@ -151,7 +174,9 @@ struct ProjRoute {
 
 inline ProjRoute proj_route(const KernelSwitches &sw, int path, int rows, int K, int N, int n_cu)
 {
-    ProjRoute r{false, proj_gemm_slices(sw, path, rows, K, N, n_cu), N};
+    const ProjGemm g = proj_gemm(sw, path, rows, K, N, n_cu);
+    ProjRoute r{false, g.ks, N};
+    if (path == DP_Q80 && g.ks && sw.proj_gemm < 0 && !q80_gemm_pays(g, rows, K, N, n_cu)) r.gemm_ks = 0;
     const bool int4_6 = path == DP_Q4K || path == DP_Q6K;
     if (int4_6 && proj_ok(rows, K, N) && (N < proj_gemm_min_tokens(path, rows) || !r.gemm_ks))
         return ProjRoute{true, 0, N};
@@ -164,7 +189,7 @@ inline ProjRoute proj_route(const KernelSwitches &sw, int path, int rows, int K,
 // GEMM does not take the shape), or the GEMM's gate/up and down launches.
 inline ProjRoute dense_route(const KernelSwitches &sw, int path, int H, int FF, int N, int n_cu)
 {
-    const int ks = path == DP_Q80 || 2L * N * H >= (1L << 31) ? 0 : proj_gemm_slices(sw, path, H, FF, N, n_cu);
+    const int ks = path == DP_Q80 || 2L * N * H >= (1L << 31) ? 0 : proj_gemm(sw, path, H, FF, N, n_cu).ks;
     const int chunk = path == DP_Q6K && !ks ? std::min(N, PROJ_MAX_TOKENS) : N;
     const bool int4_6 = path == DP_Q4K || path == DP_Q6K;
     if (int4_6 && proj_ok(FF, H, chunk) && proj_ok(H, FF, chunk)) return ProjRoute{true, 0, chunk};

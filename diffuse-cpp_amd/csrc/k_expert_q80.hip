@@ -44,6 +44,7 @@ constexpr int Q8_IT_GU = 4;                          // gate/up passes: gate, up
 constexpr int Q8_IT_DN = 2;                          // down passes: two 16-row tiles a wavefront
 constexpr int Q8_GROWS_GU = Q8_WAVES * 16 * 2;       // gate/up rows of an item: one h super-block
 constexpr int Q8_GROWS_DN = Q8_WAVES * 16 * Q8_IT_DN; // down rows
+static_assert(Q8_GROWS_DN == 256, "the item rows that q80_gemm_pays weighs");
 constexpr int Q8_STEP_ROW = 8 * Q8_0_BYTES;          // 272 bytes of a row per 256 values
 constexpr int Q8_TILE = 16 * Q8_STEP_ROW;            // 4352 bytes: one tile, one step
 constexpr int Q8_WPIECES = Q8_TILE / 16;             // 272

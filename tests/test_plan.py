@@ -95,3 +95,16 @@ def test_routed_q4k_gemm(routes, top_k, E, FF, N, block, gemm):
     measured ahead of the tile kernels: enough items, and with plain top-k
     more pairs per expert."""
     assert routes([("m", top_k, E, FF, N, block)])[0][0] == gemm
+
+
+@pytest.mark.parametrize("rows,K,N,gemm", [
+    (2048, 512, 16, 1), (1536, 512, 32, 0), (2048, 512, 64, 0), (16384, 512, 200, 1), (4096, 1024, 32, 1),
+    (4096, 1024, 48, 0),
+    (4096, 2048, 64, 1), (4096, 2816, 16, 1), (4096, 2816, 32, 0), (16384, 2816, 64, 0), (16384, 2816, 96, 1),
+    (1024, 4096, 1, 1), (4096, 4096, 512, 1), (157184, 4096, 8, 0), (157184, 4096, 9, 1)])
+def test_q80_gemm_or_items(routes, rows, K, N, gemm):
+    """Q8_0 projections: the GEMM where it measured ahead of the items of 8
+    tokens (few rows and short reductions keep those); DMOE_PROJ_GEMM pins it."""
+    ask = [("p", Q80, rows, K, N, f) for f in (-1, 0, 1)]
+    got = [r[1] > 0 for r in routes(ask)]
+    assert got == [bool(gemm), False, True]
