@@ -254,11 +254,6 @@ struct ProjJob {
     float *out;              // partial: [M][KS][N][R] slice sums; else y [N][ldo] (M = KS = 1)
     int32_t partial, ldo;
 };
-struct ProjPlan {
-    int T;                   // 16-row tiles per wavefront
-    int KS;                  // reduction slices
-};
-ProjPlan proj_plan(int R, int K, int M, int N);          // the launch shape for a projection
 size_t proj_partial_floats(int R, int K, int M, int N);  // partial buffer of that KS
 hipError_t launch_proj_q4k(const ProjJob &j, hipStream_t s);
 // the same for Q6_K matrices (tiled by launch_tile_q6k)

@@ -36,10 +36,53 @@ enum WeightPath { DP_GEMV = 0, DP_Q4K, DP_Q80, DP_F16, DP_Q6K };
 
 // The few-token kernel (k_proj.hip): Q4_K and Q6_K, up to 32 tokens a launch.
 constexpr int PROJ_MAX_TOKENS = 32;
+constexpr int PROJ_WAVES = 8, PROJ_TMAX = 6;     // wavefronts of a workgroup, 16-row tiles of a wavefront at most
+constexpr int PROJ_STEP_BYTES = 4672;            // activations of 8 tokens and a super-block
 
 inline bool proj_ok(int R, int K, int N)
 {
     return R > 0 && R % 16 == 0 && K > 0 && K % 256 == 0 && N > 0 && N <= PROJ_MAX_TOKENS;
+}
+
+// Tiles per wavefront (T) and reduction slices (KS, a divisor of K / 256)
+// for a shape, by a cost model fitted to measured launches on the 256-CU
+// part this is built for (at 32 tokens): a launch takes about 8 us plus
+// 1.9 us per tile step of a wavefront (T S) and round of workgroups over the
+// CUs, and the slices' sums, when there are several, about 2 us plus 0.6 us
+// per MB to add (k_proj_reduce / k_proj_swiglu); the activation steps every
+// workgroup reads from L2 (4.7 KB per 8 tokens and super-block) count 0.1 us
+// per MB.  Ties go to more tiles per wavefront.
+struct ProjPlan {
+    int T;                   // 16-row tiles per wavefront
+    int KS;                  // reduction slices
+    double us;               // the model's estimate
+};
+
+inline ProjPlan proj_plan(int R, int K, int M, int N)
+{
+    const int tiles = R / 16, nsb = K / 256;
+    const int nb = (N + 7) / 8;
+    ProjPlan best{1, nsb, -1.0};
+    for (int t = PROJ_TMAX; t >= 1; t--)
+        for (int ks = 1; ks <= nsb; ks++) {
+            if (nsb % ks) continue;
+            const long wgs = (long)((tiles + PROJ_WAVES * t - 1) / (PROJ_WAVES * t)) * M * ks;
+            const long rounds = (wgs + 255) / 256;
+            double us = 8.0 + 1.9 * t * (nsb / ks) * rounds;
+            if (ks > 1) us += 2.0 + 0.6 * ((double)M * ks * N * R * 4 / 1e6);
+            us += 0.1 * ((double)wgs * (nsb / ks) * nb * PROJ_STEP_BYTES / 1e6);
+            if (best.us < 0.0 || us < best.us) best = ProjPlan{t, ks, us};
+        }
+    return best;
+}
+
+// Q6_K past 32 tokens in chunks of 32 of that kernel, by the model: a
+// launch and its share of the conversions take 1.1 times its estimate and 1 us.
+inline double proj_chunks_us(int R, int K, int M, int N)
+{
+    double us = N / PROJ_MAX_TOKENS ? (N / PROJ_MAX_TOKENS) * (1.1 * proj_plan(R, K, M, PROJ_MAX_TOKENS).us + 1.0) : 0.0;
+    if (const int n = N % PROJ_MAX_TOKENS) us += 1.1 * proj_plan(R, K, M, n).us + 1.0;
+    return us;
 }
 
 // Output rows up to which a few-token Q4_K projection runs one workgroup per
@@ -98,11 +141,12 @@ struct ProjGemm {
 constexpr int PROJ_GEMM_MIN_TOKENS = 33;
 
 // Q6_K matrices of an LM head's rows take the GEMM (in units of 32 tokens)
-// from 17 tokens on: at 157,184 x 4,096 rows 16 / 17 / 24 / 32 tokens 145 / 167
-// / 172 / 177 us against 140 / 174 / 177 / 217 on the few-token kernel, whose
-// work per weight grows by the eight tokens.  A few thousand rows fill too few
-// of the GEMM's 256-row items.
-constexpr int PROJ_GEMM_MIN_TOKENS_Q6K_HEAD = 17;
+// from 17 tokens on where q6k_head_gemm_pays says so, from 25 on always: the
+// few-token kernel's work per weight grows by the eight tokens, the GEMM's not.
+// Few-token kernel against GEMM at 25 / 32 tokens, us: 157,184 x 4,096 220 / 224 against
+// 177 / 182, 157,184 x 2,048 121 / 123 against 107 / 103, 33,024 x 2,048 51 / 54
+// against 46 / 48.
+constexpr int PROJ_GEMM_MIN_TOKENS_Q6K_HEAD = 17, PROJ_GEMM_ANY_TOKENS_Q6K_HEAD = 25;
 
 // Q8_0 projections have no few-token kernel of their own: against the expert
 // kernel's items of 8 tokens the GEMM takes the attention half of 1 / 8 / 20
@@ -159,6 +203,39 @@ inline bool q80_gemm_pays(const ProjGemm &g, int rows, int K, int N, int n_cu)
     return gemm_us <= 2.2 * nsb * (double)((items + grid - 1) / grid) + 1.0;
 }
 
+// A Q6_K head of 17 to 24 tokens: a step of the GEMM's units of 32 tokens
+// lasts about 3.55 us, its slices an own launch and their traffic; the few-token
+// kernel takes nine tenths of its estimate.  Over 135 measured heads (33,024 to 157,184 rows x
+// 1,024 to 5,120) never the slower by more than 1 percent.  Few-token kernel against
+// GEMM at 20 tokens, us: 65,536 x 4,096 85 against 71, 100,352 x 2,048 81 against
+// 70 (the GEMM); 157,184 x 2,048 101 against 104, 81,920 x 1,024 43 against 47 (row groups that
+// leave its last round half empty, or the slices' launch on a short
+// reduction).
+inline bool q6k_head_gemm_pays(const ProjGemm &g, int rows, int K, int N)
+{
+    double gemm_us = 3.55 * (double)(g.rounds * (K / 256 / g.ks));
+    if (g.ks > 1) gemm_us += 6.0 + (double)g.ks * N * rows * 8 / 4e6;
+    return gemm_us <= 0.9 * proj_plan(rows, K, 1, N).us;
+}
+
+// Q6_K past the few-token kernel: the GEMM (gemm_us) against chunks of 32 tokens
+// of that kernel.  They read the matrix again for every chunk but split a
+// reduction by any divisor, the GEMM by powers of two: with an odd number of
+// super-blocks a workgroup walks all of them (4.5 us each) however few rows
+// there are.  Over 270 projections (512 to 16,384 rows x 512 to 4,096, 33 to
+// 160 tokens) the rule never picks the slower; chunks against GEMM, us:
+// 1,024 x 2,816 at 33 / 65 / 160 tokens 37 / 52 / 84 against 54 / 58 / 59, 8,192 x 2,816 at
+// 33 / 64 52 / 63 against 55 / 58, 1,024 x 4,096 at 33 40 against 28.  Dense
+// MLPs, 175 shapes: 4,096 x 11,008 at 33 / 65 tokens 181 / 257 against 215 / 225, 1,024 x
+// 2,816 at 64 56 against 73, 4,096 x 9,216 at 33 140 against 107.
+template <class ChunksUs>
+bool q6k_gemm_pays(double gemm_us, int N, ChunksUs &&chunks_us)
+{
+    // (the model is asked only when it can matter: no chunk's estimate is below 11.8 us)
+    const int chunks = (N + PROJ_MAX_TOKENS - 1) / PROJ_MAX_TOKENS;
+    return gemm_us <= 11.8 * chunks || gemm_us <= chunks_us();
+}
+
 // What a projection y [N][rows] = W x, or a dense MLP, runs on:
 //   few          the few-token kernel, `chunk` tokens a launch (Q6_K of any N:
 //                it has no item kernel; Q4_K in one launch)
@@ -177,6 +254,12 @@ inline ProjRoute proj_route(const KernelSwitches &sw, int path, int rows, int K,
     const ProjGemm g = proj_gemm(sw, path, rows, K, N, n_cu);
     ProjRoute r{false, g.ks, N};
     if (path == DP_Q80 && g.ks && sw.proj_gemm < 0 && !q80_gemm_pays(g, rows, K, N, n_cu)) r.gemm_ks = 0;
+    if (path == DP_Q6K && g.ks && sw.proj_gemm < 0 && N > PROJ_MAX_TOKENS &&
+        !q6k_gemm_pays(g.us + (g.ks > 1 ? 2.0 : 0.0), N, [&] { return proj_chunks_us(rows, K, 1, N); }))
+        r.gemm_ks = 0;
+    if (path == DP_Q6K && g.ks && sw.proj_gemm < 0 && N < PROJ_GEMM_ANY_TOKENS_Q6K_HEAD &&
+        !q6k_head_gemm_pays(g, rows, K, N))
+        r.gemm_ks = 0;
     const bool int4_6 = path == DP_Q4K || path == DP_Q6K;
     if (int4_6 && proj_ok(rows, K, N) && (N < proj_gemm_min_tokens(path, rows) || !r.gemm_ks))
         return ProjRoute{true, 0, N};
@@ -186,10 +269,18 @@ inline ProjRoute proj_route(const KernelSwitches &sw, int path, int rows, int K,
 
 // The dense MLP: gate and up as one two-matrix projection and down as
 // another, both on the few-token kernel (Q6_K past it in chunks, where the
-// GEMM does not take the shape), or the GEMM's gate/up and down launches.
+// GEMM does not take the shape or is slower), or the GEMM's gate/up and down launches.
 inline ProjRoute dense_route(const KernelSwitches &sw, int path, int H, int FF, int N, int n_cu)
 {
-    const int ks = path == DP_Q80 || 2L * N * H >= (1L << 31) ? 0 : proj_gemm(sw, path, H, FF, N, n_cu).ks;
+    const ProjGemm g = proj_gemm(sw, path, H, FF, N, n_cu);
+    int ks = path == DP_Q80 || 2L * N * H >= (1L << 31) ? 0 : g.ks;
+    if (path == DP_Q6K && ks && sw.proj_gemm < 0 && N > PROJ_MAX_TOKENS) {
+        const long grid = (n_cu + 7) / 8 * 8, items = (long)((N + 63) / 64) * (FF / EXPERT_GEMM_GU_ROWS);
+        const double gu_us = 4.5 * (double)((items + grid - 1) / grid * (H / 256));
+        if (!q6k_gemm_pays(gu_us + g.us + (ks > 1 ? 2.0 : 0.0), N,
+                           [&] { return proj_chunks_us(FF, H, 2, N) + proj_chunks_us(H, FF, 1, N); }))
+            ks = 0;
+    }
     const int chunk = path == DP_Q6K && !ks ? std::min(N, PROJ_MAX_TOKENS) : N;
     const bool int4_6 = path == DP_Q4K || path == DP_Q6K;
     if (int4_6 && proj_ok(FF, H, chunk) && proj_ok(H, FF, chunk)) return ProjRoute{true, 0, chunk};

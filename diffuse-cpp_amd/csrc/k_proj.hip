@@ -33,11 +33,12 @@
 
 namespace dmoe {
 
-constexpr int PJ_WAVES = 8;                       // wavefronts of a workgroup
+constexpr int PJ_WAVES = PROJ_WAVES;              // wavefronts of a workgroup
 constexpr int PJ_BLOCKS = PROJ_MAX_TOKENS / 8;    // column blocks of 8 tokens
 constexpr int PJ_WST = 5;                         // weight ring stages per wavefront
 constexpr int PJ_AHEAD = PJ_WST - 1;              // tile steps in flight
-constexpr int PJ_TMAX = 6;                        // tiles per wavefront at most
+constexpr int PJ_TMAX = PROJ_TMAX;                // tiles per wavefront at most
+static_assert(PROJ_STEP_BYTES == ASTEP_BYTES, "the activation step that proj_plan weighs");
 
 // s_waitcnt vmcnt(n), lgkmcnt(0) for a compile-time n below 64 (vmcnt bits
 // 5:4 at 15:14)
@@ -582,36 +583,6 @@ __global__ __launch_bounds__(256) void k_proj_swiglu(const float *__restrict__ p
         v[c] = silu(gsum) * usum;
     }
     prep_values(v, ah, ACT_SPLIT, t, N, sb, nsb, s_v[w]);
-}
-
-// Tiles per wavefront (T) and reduction slices (KS, a divisor of K / 256)
-// for a shape, by a cost model fitted to measured launches on the 256-CU
-// part this is built for (at 32 tokens): a launch takes about 8 us plus
-// 1.9 us per tile step of a wavefront (T S) and round of workgroups over the
-// CUs, and the slices' sums, when there are several, about 2 us plus 0.6 us
-// per MB to add (k_proj_reduce / k_proj_swiglu); the activation steps every
-// workgroup reads from L2 (4.7 KB per 8 tokens and super-block) count 0.1 us
-// per MB.  Ties go to more tiles per wavefront.
-ProjPlan proj_plan(int R, int K, int M, int N)
-{
-    const int tiles = R / 16, nsb = K / 256;
-    const int nb = (N + 7) / 8;
-    ProjPlan best{1, nsb};
-    double best_us = -1.0;
-    for (int t = PJ_TMAX; t >= 1; t--)
-        for (int ks = 1; ks <= nsb; ks++) {
-            if (nsb % ks) continue;
-            const long wgs = (long)((tiles + PJ_WAVES * t - 1) / (PJ_WAVES * t)) * M * ks;
-            const long rounds = (wgs + 255) / 256;
-            double us = 8.0 + 1.9 * t * (nsb / ks) * rounds;
-            if (ks > 1) us += 2.0 + 0.6 * ((double)M * ks * N * R * 4 / 1e6);
-            us += 0.1 * ((double)wgs * (nsb / ks) * nb * ASTEP_BYTES / 1e6);
-            if (best_us < 0.0 || us < best_us) {
-                best_us = us;
-                best = ProjPlan{t, ks};
-            }
-        }
-    return best;
 }
 
 size_t proj_partial_floats(int R, int K, int M, int N)

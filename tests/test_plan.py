@@ -108,3 +108,21 @@ def test_q80_gemm_or_items(routes, rows, K, N, gemm):
     ask = [("p", Q80, rows, K, N, f) for f in (-1, 0, 1)]
     got = [r[1] > 0 for r in routes(ask)]
     assert got == [bool(gemm), False, True]
+
+
+@pytest.mark.parametrize("kind,rows,K,N,gemm", [
+    # heads of 17 to 24 tokens by the model, from 25 on always
+    ("p", 157184, 4096, 16, 0), ("p", 157184, 2048, 17, 0), ("p", 157184, 2048, 24, 0), ("p", 157184, 2048, 25, 1),
+    ("p", 65536, 4096, 17, 1), ("p", 100352, 2048, 20, 1), ("p", 81920, 1024, 20, 0), ("p", 33024, 2048, 17, 0),
+    # past 32 tokens: an odd number of super-blocks is one slice
+    ("p", 1024, 2816, 33, 0), ("p", 1024, 2816, 65, 0), ("p", 1024, 2816, 160, 1), ("p", 16384, 2816, 33, 1),
+    ("p", 1024, 4096, 32, 0), ("p", 1024, 4096, 33, 1), ("p", 512, 512, 33, 1),
+    # dense MLPs (n_embd, n_ff)
+    ("d", 4096, 11008, 33, 0), ("d", 4096, 11008, 200, 1), ("d", 1024, 2816, 64, 0), ("d", 1024, 2816, 200, 1),
+    ("d", 4096, 9216, 33, 1), ("d", 512, 1536, 33, 1)])
+def test_q6k_gemm_or_chunks(routes, kind, rows, K, N, gemm):
+    """Q6_K: the grouped GEMM where it measured ahead of the few-token kernel
+    and its chunks of 32 tokens; DMOE_PROJ_GEMM = 0 keeps those."""
+    (few, ks, chunk), off = routes([(kind, Q6K, rows, K, N, f) for f in (-1, 0)])
+    assert (few, ks > 0, chunk) == ((0, True, N) if gemm else (1, False, min(N, 32)))
+    assert off == (1, 0, min(N, 32))
