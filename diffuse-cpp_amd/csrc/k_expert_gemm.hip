@@ -551,6 +551,7 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
         auto run = [&](auto nb_c, auto half_c) __attribute__((always_inline)) {
             constexpr int NB = decltype(nb_c)::value;
             constexpr bool HALF = decltype(half_c)::value;
+            static_assert(NB + HALF <= NBMAX, "the accumulators of a unit");
             for (int s = 0; s < steps; s++) {
                 // this step's weights (this wavefront's) and activations
                 // (every wavefront's) have landed, the stage two steps on has
@@ -813,7 +814,13 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
         };
         typedef std::integral_constant<int, 0> zero;
         typedef std::integral_constant<int, 1> one;
-        if constexpr (MERGE) {
+        if constexpr (FEW) {
+            // (32 tokens at most: half a block or a whole one)
+            if (I.nblk >> 1 == 1)
+                run(zero(), one());
+            else
+                run(one(), zero());
+        } else if constexpr (MERGE) {
             switch (I.nblk >> 1) {
             case 1: run(zero(), one()); break;
             case 2: run(one(), zero()); break;
