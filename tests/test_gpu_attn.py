@@ -158,7 +158,7 @@ def test_attn_rejects(ctx, O):
 def test_attn_flash_q6k(ctx, O, N):
     """The flash-shaped attention half with Q6_K projections (the q6_k
     scheme's attn tensors): 32 tokens through the fused norm and few-token
-    kernel, 96 in chunks of 32."""
+    kernel, 96 through the fused norm and the grouped GEMM."""
     from dmoe import synth
     _say(f"case: attn flash shape Q6_K N={N}")
     w = synth.host_attn(14, 6, O.quantize_rows, **synth.ATTN_FLASH)

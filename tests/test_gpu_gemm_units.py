@@ -34,8 +34,8 @@ def test_head_units(ctx, O, wtype, N):
 
 @pytest.mark.parametrize("N", [1, 7, 16, 17, 32])
 def test_head_q80_few_tokens(ctx, O, N):
-    """Q8_0 projections take the GEMM at any token count (half blocks, one
-    token), unless they are an LM head's."""
+    """Q8_0 projections of few tokens on the GEMM (half blocks, one token):
+    this shape takes it at each of these counts."""
     from dmoe import synth
     H, V = 1024, 1280
     print(f"case: LM head H={H} V={V} Q8_0 N={N}", flush=True)

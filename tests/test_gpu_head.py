@@ -64,7 +64,8 @@ def test_head_small(ctx, O, wtype, N):
 def test_head_q4k_column_blocks(ctx, O, N, wtype):
     """The few-token projection at each column-block count (1 to 4 blocks of
     8 tokens, the last one partly filled), Q4_K and Q6_K, against the
-    oracle; 72 tokens: Q6_K in chunks of 32, 32 and 8 tokens."""
+    oracle; 72 tokens: the grouped GEMM (test_gpu_q6k_chunks runs the chunks of
+    32 tokens)."""
     from dmoe import synth
     H, V = 512, 4096
     _say(f"case: step tail type={wtype} H={H} V={V} N={N}")

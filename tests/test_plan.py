@@ -126,3 +126,18 @@ def test_q6k_gemm_or_chunks(routes, kind, rows, K, N, gemm):
     (few, ks, chunk), off = routes([(kind, Q6K, rows, K, N, f) for f in (-1, 0)])
     assert (few, ks > 0, chunk) == ((0, True, N) if gemm else (1, False, min(N, 32)))
     assert off == (1, 0, min(N, 32))
+
+
+def test_routes_of_the_gpu_tests(routes):
+    """What GPU tests say of their shapes: the projection of the rotary step's
+    slices, the Q6_K chunks, the Q8_0 heads of few tokens."""
+    assert routes([("p", Q4K, 4096, 2048, 1030, -1)]) == [(0, 2, 1030)]
+    chunks = [("d", Q6K, 256, 768, 72, -1), ("d", Q6K, 768, 256, 72, -1), ("d", Q6K, 512, 2816, 64, -1)]
+    chunks += [("p", Q6K, 1296, 512, 72, -1), ("p", Q6K, 1280, 256, 72, -1), ("p", Q6K, 1024, 2816, 72, -1)]
+    assert all(r == (1, 0, 32) for r in routes(chunks))
+    gemm = [("p", Q80, 1280, 1024, n, -1) for n in (1, 7, 16, 17, 32)] + [("p", Q6K, 4096, 512, 72, -1)]
+    gemm += [("p", Q6K, 33024, K, n, -1) for K in (512, 1024) for n in (17, 31, 32)]
+    gemm += [("p", Q6K, 5120, 4096, 96, -1), ("p", Q6K, 4096, 4096, 96, -1)]
+    gemm += [("d", Q6K, 1024, 1536, n, -1) for n in (33, 64, 90, 129)]
+    gemm += [("p", Q6K, 1280, 512, n, -1) for n in (33, 48, 63, 64, 65, 97, 128)]
+    assert all(r[1] > 0 for r in routes(gemm))
