@@ -133,7 +133,7 @@ def uses_tile_kernels(cfg):
 def uses_q4k_gemm(cfg):
     """Whether the library runs cfg's Q4_K expert products on its grouped
     GEMM (k_expert_gemm.hip): the rule of use_q4k_gemm in dmoe_api.cpp for
-    the flash shapes (32 or more pairs per expert averaged over all experts,
+    the flash shapes in whole blocks (32 or more pairs per expert over all experts,
     N k / E), DMOE_EXPERT_GEMM overriding it and DMOE_EXPERT_TILE turning it
     off."""
     import dmoe

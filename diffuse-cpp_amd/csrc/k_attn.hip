@@ -40,7 +40,11 @@ constexpr int QR_THREADS = 256;
 // the launch of 2,048 tokens of 40 heads leaves the attention half at 580 us
 // against 591.  Fewer rows need the wavefronts: 777 tokens 243 us either way,
 // 256 tokens 105 against 102 (eight heads: 581, 251, 112 us); one head per
-// wavefront by that kernel takes 48.0 us at 32 tokens against 47.3.
+// wavefront by that kernel takes 48.0 us at 32 tokens against 47.3.  In between, one head
+// against four: 36,000 rows 279 / 281 us, 40,960 294 / 294, 51,200 403 / 397, 61,440
+// 470 / 463 (of 40 heads), 65,600 542 / 541 (a projection in two slices), 81,920
+// 577 / 569; 40,968 rows of 24 heads 261 / 257.  The line stays where it is ahead
+// in every shape measured.
 constexpr int QR_HEADS = 4;
 constexpr long QR_MANY = 65536;
 

@@ -15,10 +15,16 @@
 // (schedule_item): with row groups a multiple of 8 per unit, one row group of
 // every unit runs on one XCD (workgroup b is placed on XCD b % 8) and
 // consecutive units together, so chunks of one expert next to each other read
-// its weights once from HBM and then from that XCD's L2.  The units go out by
-// falling size, the shared ones first, then the work list (by_size): at 2,048
-// tokens a CU runs about seven units of one to eight blocks, and in expert
-// order a wavefront was busy for 0.76 (gate/up) of the launch.
+// its weights once from HBM and then from that XCD's L2 (four row groups, the
+// gate/up units of moe_ff 512, alternate between two XCDs, so such a row group
+// is read twice).  The units go out by falling size, the shared ones first,
+// then the work list (by_size): at 2,048 tokens a CU runs about seven units of
+// one to eight blocks, and in expert order a wavefront was busy for 0.76
+// (gate/up) of the launch.  That order costs the combine launch after it,
+// which finds less of the products in the last-level cache.  2,048 tokens, each
+// pass alone, us, expert order and shared units last / by size, shared last /
+// by size, shared first: gate/up 556 / 501 / 502, down 311 / 305 / 303, combine
+// 61 / 66 / 70, the layer 1,058 / 1,033 / 1,040; 1,024 tokens 613 / 599 / 589.
 //
 // Pipeline: one step per 256-value super-block of the reduction.  A
 // wavefront's 32 weight rows are private to it: one LDS buffer of their own
@@ -32,29 +38,34 @@
 // Products: v_mfma_i32_32x32x32_i8 on 32 activation rows x 32 weight rows.
 // The sub-block scales are folded into the int8 weight operand once per step
 // (sc = 8 sh + sl, sh and sl below 8: sh q and sl q are int8) and applied to
-// all the unit's rows.  What bounds a step is the SIMD's issue and, in steady
-// state, the power that issue takes: per 32 x 32 output tile and super-block 16
-// int8 MFMAs of 32 cycles (twice the useful products: the two scale digits; 44
-// cycles each in steady state on such operands), 80 VALU instructions of scale
+// all the unit's rows.  What bounds a step is the SIMD's issue and, in large
+// calls that run on end, the clock that issue leaves (below): per 32 x 32 output
+// tile and super-block 16 int8 MFMAs of 32 cycles (twice the useful products:
+// the two scale digits), 80 VALU instructions of scale
 // epilogue (five per output) and the fold's ~150 shared by up to four tiles.
 // Launches with shared units only (MERGE) keep a token's two digit rows in
 // separate blocks of 32, so that both digits of an output lie in one lane and
 // take one epilogue (8 instructions per token against 10).
 //
-// Measured (steady state, the card at its power limit, against 16 x 16 MFMA
-// tiles with one epilogue per digit row, the weights and activations of a step
-// in one of two shared stages, units in expert order): Q4_K MoE layer of 2,048
-// tokens 1,073 -> 1,012 us, of 1,024 tokens 646 -> 582; dense MLP of 160 tokens
-// 129 -> 110 us, of 512 314 -> 286; attention half of 777 tokens 268 -> 247, of
-// 2,048 612 -> 603 us.  In bursts too short to reach the power limit the MoE
-// launches gain more (620 -> 497 and 314 -> 300 us at 2,048 tokens, mostly the
-// schedule); in steady state an even schedule buys less, since busy CUs run
-// faster while others wait.
+// Measured (calls on end, against 16 x 16 MFMA tiles with one epilogue per
+// digit row, the weights and activations of a step in one of two shared stages,
+// units in expert order): Q4_K MoE layer of 2,048 tokens 1,073 -> 1,012 us, of
+// 1,024 tokens 646 -> 582; dense MLP of 160 tokens 129 -> 110 us, of 512 314 ->
+// 286; attention half of 777 tokens 268 -> 247, of 2,048 612 -> 603 us.  In
+// calls on end the card lowers its clock under the large ones: MoE layer of
+// 2,048 tokens 2,146 MHz (2,398 with the former tiles), attention half of 2,048
+// 2,312 (2,400), Q6_K head of 256 tokens 1,968; the dense MLP of 160 tokens stays at
+// 2,398.  The launches around the GEMM slow down with it, so the layer gains less than
+// the launches do in short runs (620 -> 497 and 314 -> 300 us at 2,048 tokens).
 //
 // Arithmetic: the integer sums of every super-block are compute_sb's exactly
 // (8 sum (sh q) a + sum (sl q) a = sum_j sc_j S_j), then one f32 epilogue per
-// super-block in super-block order rounded by q4k_epi, so the outputs equal
-// the tile and column-block kernels' bit for bit.  h goes to HBM as f32
+// super-block in super-block order rounded by q4k_epi, so the outputs of routed
+// launches equal the tile and column-block kernels' bit for bit.  MERGE
+// launches round a token's two digits together, in a full block of 32 tokens
+// also the min term's sum (past 2^24, in the MFMA's accumulation), in a half
+// block that sum's two parts by one fused multiply-add: a token's last bits depend on
+// the block it falls in, as on the reduction's slices.  h goes to HBM as f32
 // ([pair][moe_ff], [token][shared_ff]) and one conversion launch writes the
 // down products' int8 layout; the down products go to ye [pair][n_embd] /
 // ys [token][n_embd] for the combine launch, as with the tile kernels.
@@ -699,7 +710,8 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
                             if constexpr (F::MIN)
                                 if (i == 6) {
                                     // sums of 16: 256 (a1 sums) + (a0 sums), the
-                                    // factor on the operand (m <= 63: exact)
+                                    // factor on the operand (m <= 63: exact
+                                    // there; the f32 sum may round)
                                     const h8 s1 = *reinterpret_cast<const h8 *>(ab1 + XG_ABS + r32 * 32 + 16 * h);
                                     const h8 s0 = *reinterpret_cast<const h8 *>(ab0 + XG_ABS + r32 * 32 + 16 * h);
                                     s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(s1, f.bm * (_Float16)256.0f, s2, 0, 0, 0);
@@ -916,7 +928,7 @@ __global__ __launch_bounds__(XG_WAVES * 64) void k_gemm_q(MoeJob job)
 }
 
 // ---------------------------------------------------------------------------
-// One workgroup per CU (the two stages fill the LDS), a multiple of 8 (one
+// One workgroup per CU (the activation ring and the weight buffers fill the LDS), a multiple of 8 (one
 // row group per XCD); each runs its items until the schedule's units end.
 hipError_t launch_expert_gemm_q4k(int phase, const MoeJob &job, hipStream_t s)
 {
