@@ -1100,7 +1100,8 @@ struct DenseWs {
     ActI8 axs, ahs;                      // split x and h (int8 paths)
     uint16_t *xs16, *hs16;               // hi / lo f16 pairs (F16 path)
     float *hs;                           // f32 h (GEMV path)
-    float *part_gu, *part_d;             // slice sums of the few-token Q4_K projections
+    float *part_gu, *part_d;             // slice sums of the few-token projections or the GEMM
+    ProjRoute route;                     // what the workspace is planned for and the launches take
 };
 
 // Slice-sum floats the few-token projection of R x K (M matrices) needs at
@@ -1151,15 +1152,15 @@ size_t plan_dense(const KernelSwitches &sw, const dmoe_layer *L, int N, bool hos
     }
     t.n_ec = (int32_t *)take(4);
     const int path = dense_path(L->sg.type, H, FF);
+    t.route = dense_route(sw, path, H, FF, N, plan_cus());
     switch (path) {
     case DP_Q4K:
     case DP_Q6K: {
         // Q6_K in chunks: workspace for one, reused chunk after chunk
-        const ProjRoute r = dense_route(sw, path, H, FF, N, plan_cus());
-        const int n = r.chunk, ks = r.gemm_ks;
+        const int n = t.route.chunk, ks = t.route.gemm_ks;
         t.axs = take_act(take, n, H, true);
         t.ahs = take_act(take, n, FF, true);
-        if (r.few) {
+        if (t.route.few) {
             t.part_gu = (float *)take(proj_partial_max(FF, H, 2, n, false) * 4);
             if (const size_t pd = proj_partial_max(H, FF, 1, n, true)) t.part_d = (float *)take(pd * 4);
         } else if (ks) {
@@ -1204,9 +1205,8 @@ int ensure_dense_workspace(dmoe_ctx *ctx, const dmoe_layer *L, int N, bool host_
     return DMOE_OK;
 }
 
-// sw: the switches that w was planned with
-int enqueue_dense(dmoe_ctx *ctx, const KernelSwitches &sw, const dmoe_layer *L, const DenseWs &w, const float *x,
-                  int N, float *y, hipStream_t s, bool prof)
+int enqueue_dense(dmoe_ctx *ctx, const dmoe_layer *L, const DenseWs &w, const float *x, int N,
+                  float *y, hipStream_t s, bool prof)
 {
     const int H = L->hp.n_embd, FF = L->hp.shared_ff;
     const int path = dense_path(L->sg.type, H, FF);
@@ -1216,12 +1216,11 @@ int enqueue_dense(dmoe_ctx *ctx, const KernelSwitches &sw, const dmoe_layer *L, 
         STAGE(ST_SH_DOWN, launch_down_shared(L->sd, w.hs, N, FF, H, y, s));
         return DMOE_OK;
     }
-    const ProjRoute r = dense_route(sw, path, H, FF, N, plan_cus());
-    if (r.few) {
+    if (w.route.few) {
         // gate and up: one launch over both matrices, h from their slices;
         // tokens t0 .. t0 + n - 1 at a time (every token at once, or Q6_K chunks)
         const bool q6 = path == DP_Q6K;
-        const int nc = r.chunk;
+        const int nc = w.route.chunk;
         for (int t0 = 0; t0 < N; t0 += nc) {
             const int n = std::min(nc, N - t0);
             ProjJob gu{};
@@ -1255,7 +1254,7 @@ int enqueue_dense(dmoe_ctx *ctx, const KernelSwitches &sw, const dmoe_layer *L, 
         }
         return DMOE_OK;
     }
-    if (const int ks = r.gemm_ks) {
+    if (const int ks = w.route.gemm_ks) {
         // many tokens of Q4_K or Q6_K: the grouped GEMM's gate/up and down launches
         // over shared units (no routed work list), h converted between them,
         // the down reduction in slices added in order
@@ -1333,7 +1332,7 @@ int enqueue_dense(dmoe_ctx *ctx, const KernelSwitches &sw, const dmoe_layer *L, 
     job.ys = y;                          // the shared expert's down output is the MLP's
     PrepJob pj{x, N, H, q8 ? ACT_SPLIT32 : ACT_SPLIT, w.axs};
     STAGE(ST_ACTQ_X, launch_prep(&pj, 1, s));
-    STAGE(ST_SH_GATEUP, q8 ? launch_expert_q80(0, job, s) : launch_expert_q4k(0, job, s, 1, sw.gateup_lds));
+    STAGE(ST_SH_GATEUP, q8 ? launch_expert_q80(0, job, s) : launch_expert_q4k(0, job, s, 1, ctx->sw.gateup_lds));
     STAGE(ST_SH_DOWN, q8 ? launch_expert_q80(1, job, s) : launch_expert_q4k(1, job, s));
 #undef STAGE
     return DMOE_OK;
@@ -1362,7 +1361,7 @@ struct ProjWs {
     int32_t *n_ec;                       // an empty routed work list
     ActI8 act;                           // split x (int8 paths)
     uint16_t *x16;                       // hi / lo f16 x (F16 path)
-    float *part;                         // slice sums of the few-token Q4_K projection
+    float *part;                         // slice sums of the few-token projection or the GEMM
     ProjRoute route;                     // what the workspace is planned for and the launches take
 };
 
@@ -1486,7 +1485,7 @@ int enqueue_proj(dmoe_ctx *ctx, bool prof, int st_conv, int st_prod, const WTens
         return DMOE_OK;
     }
     if (p.route.gemm_ks) {
-        // many tokens of Q4_K or Q6_K, Q8_0: the grouped GEMM's down launch over shared
+        // many tokens of Q4_K, Q6_K or Q8_0: the grouped GEMM's down launch over shared
         // units, its reduction slices added in order
         PrepJob pj{x, N, K, path == DP_Q80 ? ACT_SPLIT32 : ACT_SPLIT, p.act};
         STAGE(st_conv, launch_prep(&pj, 1, s));
@@ -2271,7 +2270,7 @@ int dmoe_layer_forward(dmoe_ctx *ctx, const dmoe_layer *L, const float *x, int32
         if (rc) return rc;
         hipStream_t s = ctx->stream;
         HIP_TRY(ctx, hipMemcpyAsync(dw.x, x, (size_t)n_tokens * H * 4, hipMemcpyHostToDevice, s));
-        if ((rc = enqueue_dense(ctx, ctx->sw, L, dw, dw.x, n_tokens, dw.y, s, ctx->prof))) return rc;
+        if ((rc = enqueue_dense(ctx, L, dw, dw.x, n_tokens, dw.y, s, ctx->prof))) return rc;
         HIP_TRY(ctx, hipMemcpyAsync(y, dw.y, (size_t)n_tokens * H * 4, hipMemcpyDeviceToHost, s));
         if (dbg && dbg->use_block_routing) *dbg->use_block_routing = 0;
         HIP_TRY(ctx, hipStreamSynchronize(s));
@@ -2304,7 +2303,7 @@ int dmoe_layer_forward_device(dmoe_ctx *ctx, const dmoe_layer *L, const float *x
         DenseWs dw;
         int rc = ensure_dense_workspace(ctx, L, n_tokens, false, &dw);
         if (rc) return rc;
-        return enqueue_dense(ctx, ctx->sw, L, dw, x_dev, n_tokens, y_dev, (hipStream_t)stream, ctx->prof);
+        return enqueue_dense(ctx, L, dw, x_dev, n_tokens, y_dev, (hipStream_t)stream, ctx->prof);
     }
     Workspace w;
     int rc = ensure_workspace(ctx, L, n_tokens, false, &w);
@@ -2350,7 +2349,7 @@ int dmoe_layer_forward_device_noalloc(dmoe_ctx *ctx, const dmoe_layer *L, const 
     if (L->dense) {
         DenseWs dw;
         plan_dense(sw, L, n_tokens, false, ctx->scratch, &dw);
-        return enqueue_dense(ctx, sw, L, dw, x_dev, n_tokens, y_dev, (hipStream_t)stream, false);
+        return enqueue_dense(ctx, L, dw, x_dev, n_tokens, y_dev, (hipStream_t)stream, false);
     }
     Workspace w;
     plan_workspace(ctx->sw, L->hp, L->eg.type, L->sg.type, L->has_shared, n_tokens, false, ctx->scratch, &w);

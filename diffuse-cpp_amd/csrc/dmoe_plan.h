@@ -80,9 +80,9 @@ inline ProjPlan proj_plan(int R, int K, int M, int N)
 // launch and its share of the conversions take 1.1 times its estimate and 1 us.
 inline double proj_chunks_us(int R, int K, int M, int N)
 {
-    double us = N / PROJ_MAX_TOKENS ? (N / PROJ_MAX_TOKENS) * (1.1 * proj_plan(R, K, M, PROJ_MAX_TOKENS).us + 1.0) : 0.0;
-    if (const int n = N % PROJ_MAX_TOKENS) us += 1.1 * proj_plan(R, K, M, n).us + 1.0;
-    return us;
+    auto chunk_us = [&](int n) { return 1.1 * proj_plan(R, K, M, n).us + 1.0; };
+    const int whole = N / PROJ_MAX_TOKENS, rest = N % PROJ_MAX_TOKENS;
+    return (whole ? whole * chunk_us(PROJ_MAX_TOKENS) : 0.0) + (rest ? chunk_us(rest) : 0.0);
 }
 
 // Output rows up to which a few-token Q4_K projection runs one workgroup per
