@@ -229,8 +229,10 @@ inline bool q6k_head_gemm_pays(const ProjGemm &g, int rows, int K, int N)
 // 160 tokens) the rule never picks the slower; chunks against GEMM, us:
 // 1,024 x 2,816 at 33 / 65 / 160 tokens 37 / 52 / 84 against 54 / 58 / 59, 8,192 x 2,816 at
 // 33 / 64 52 / 63 against 55 / 58, 1,024 x 4,096 at 33 40 against 28.  Dense
-// MLPs, 175 shapes: 4,096 x 11,008 at 33 / 65 tokens 181 / 257 against 215 / 225, 1,024 x
-// 2,816 at 64 56 against 73, 4,096 x 9,216 at 33 140 against 107.
+// MLPs, 175 shapes, nowhere more than 3 percent behind the chunks: 4,096 x 11,008 at
+// 33 tokens 181 against 215, 1,024 x 2,816 at 64 56 against 73, 4,096 x 9,216 at 33 140
+// against 107 (six shapes, mostly n_ff 11,008 at 65 to 192 tokens, keep the chunks where the
+// GEMM would be 10 to 30 percent ahead).
 template <class ChunksUs>
 bool q6k_gemm_pays(double gemm_us, int N, ChunksUs &&chunks_us)
 {
