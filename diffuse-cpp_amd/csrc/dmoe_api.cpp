@@ -360,13 +360,6 @@ bool use_gemm_path(const dmoe_hparams &hp, int32_t wtype, int32_t stype, bool sh
 // DMOE_Q4K_COLUMN_BLOCKS set selects their kernels.
 bool block_routed(const dmoe_hparams &hp, int N);
 
-// The compute units the routes are planned for (without a device: a whole chip).
-int plan_cus()
-{
-    int n_cu = 0;
-    return device_cu_count(&n_cu) == hipSuccess ? n_cu : 256;
-}
-
 bool use_q4k_gemm(const KernelSwitches &sw, const dmoe_hparams &hp, int32_t wtype, int32_t stype, bool shared,
                   int N)
 {
@@ -377,7 +370,7 @@ bool use_q4k_gemm(const KernelSwitches &sw, const dmoe_hparams &hp, int32_t wtyp
     if (sw.expert_gemm >= 0) return sw.expert_gemm == 1;
     if (sw.expert_tile >= 0 || sw.q4k_column_blocks) return false;
     return moe_gemm_pays(N, hp.top_k, hp.n_experts, hp.moe_ff, shared, block_routed(hp, N),
-                         expert_tile_ok(hp.n_embd, hp.moe_ff, hp.shared_ff, shared), plan_cus());
+                         expert_tile_ok(hp.n_embd, hp.moe_ff, hp.shared_ff, shared), sw.n_cu);
 }
 
 bool use_tile_path(const KernelSwitches &sw, const dmoe_hparams &hp, int32_t wtype, int32_t stype, bool shared,
@@ -1152,7 +1145,7 @@ size_t plan_dense(const KernelSwitches &sw, const dmoe_layer *L, int N, bool hos
     }
     t.n_ec = (int32_t *)take(4);
     const int path = dense_path(L->sg.type, H, FF);
-    t.route = dense_route(sw, path, H, FF, N, plan_cus());
+    t.route = dense_route(sw, path, H, FF, N);
     switch (path) {
     case DP_Q4K:
     case DP_Q6K: {
@@ -1370,7 +1363,7 @@ ProjWs plan_proj(const KernelSwitches &sw, int path, int N, int K, int rows, Tak
 {
     ProjWs p{};
     p.n_ec = (int32_t *)take(4);
-    p.route = proj_route(sw, path, rows, K, N, plan_cus());
+    p.route = proj_route(sw, path, rows, K, N);
     const int n = p.route.chunk, ks = p.route.gemm_ks;
     switch (path) {
     case DP_Q4K:
@@ -1835,7 +1828,7 @@ int dmoe_create(int hip_device, dmoe_ctx **out)
     ctx->device = hip_device;
     ctx->sw = read_kernel_switches();
     if (hip_device >= kMaxDevices || hipSetDevice(hip_device) != hipSuccess ||
-        scratch_address(hip_device, &ctx->scratch) != hipSuccess ||
+        device_cu_count(&ctx->sw.n_cu) != hipSuccess || scratch_address(hip_device, &ctx->scratch) != hipSuccess ||
         hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
         delete ctx;
         return DMOE_ERR_HIP;

@@ -29,6 +29,7 @@ struct KernelSwitches {
     int attn_waves = 0;                  // 0: by grid size, else 4 or 8 per workgroup
     bool down_fused = false;
     bool gateup_lds = false;
+    int n_cu = 256;                      // compute units of the context's device (not a switch)
 };
 
 // Kernel family of a matrix, by its type and shape (dense_path, head_path).
@@ -162,7 +163,7 @@ inline int proj_gemm_min_tokens(int path, int rows)
     return path == DP_Q6K && rows > PROJ_ROWS_MAX ? PROJ_GEMM_MIN_TOKENS_Q6K_HEAD : PROJ_GEMM_MIN_TOKENS;
 }
 
-inline ProjGemm proj_gemm(const KernelSwitches &sw, int path, int rows, int K, int N, int n_cu)
+inline ProjGemm proj_gemm(const KernelSwitches &sw, int path, int rows, int K, int N)
 {
     ProjGemm g{0, 0, 0.0};
     if ((path != DP_Q4K && path != DP_Q6K && path != DP_Q80) || sw.proj_gemm == 0 ||
@@ -171,7 +172,7 @@ inline ProjGemm proj_gemm(const KernelSwitches &sw, int path, int rows, int K, i
         return g;
     const long items = (long)((N + 63) / 64) * (rows / 256);
     const int nsb = K / 256;
-    const long grid = (n_cu + 7) / 8 * 8;
+    const long grid = (sw.n_cu + 7) / 8 * 8;
     // rounds of the static schedule x super-blocks per item at ~4.5 us per
     // step, plus the slices written and read again at ~4 TB/s.  (A step of a
     // full unit measures 3.5 us of Q4_K, 4.4 of Q6_K, 5 of Q8_0, less of part
@@ -254,11 +255,11 @@ struct ProjRoute {
     int chunk;
 };
 
-inline ProjRoute proj_route(const KernelSwitches &sw, int path, int rows, int K, int N, int n_cu)
+inline ProjRoute proj_route(const KernelSwitches &sw, int path, int rows, int K, int N)
 {
-    const ProjGemm g = proj_gemm(sw, path, rows, K, N, n_cu);
+    const ProjGemm g = proj_gemm(sw, path, rows, K, N);
     ProjRoute r{false, g.ks, N};
-    if (path == DP_Q80 && g.ks && sw.proj_gemm < 0 && !q80_gemm_pays(g, rows, K, N, n_cu)) r.gemm_ks = 0;
+    if (path == DP_Q80 && g.ks && sw.proj_gemm < 0 && !q80_gemm_pays(g, rows, K, N, sw.n_cu)) r.gemm_ks = 0;
     if (path == DP_Q6K && g.ks && sw.proj_gemm < 0 && N > PROJ_MAX_TOKENS &&
         !q6k_gemm_pays(g.us + (g.ks > 1 ? 2.0 : 0.0), N, [&] { return proj_chunks_us(rows, K, 1, N); }))
         r.gemm_ks = 0;
@@ -275,12 +276,12 @@ inline ProjRoute proj_route(const KernelSwitches &sw, int path, int rows, int K,
 // The dense MLP: gate and up as one two-matrix projection and down as
 // another, both on the few-token kernel (Q6_K past it in chunks, where the
 // GEMM does not take the shape or is slower), or the GEMM's gate/up and down launches.
-inline ProjRoute dense_route(const KernelSwitches &sw, int path, int H, int FF, int N, int n_cu)
+inline ProjRoute dense_route(const KernelSwitches &sw, int path, int H, int FF, int N)
 {
-    const ProjGemm g = proj_gemm(sw, path, H, FF, N, n_cu);
+    const ProjGemm g = proj_gemm(sw, path, H, FF, N);
     int ks = path == DP_Q80 || 2L * N * H >= (1L << 31) ? 0 : g.ks;
     if (path == DP_Q6K && ks && sw.proj_gemm < 0 && N > PROJ_MAX_TOKENS) {
-        const long grid = (n_cu + 7) / 8 * 8, items = (long)((N + 63) / 64) * (FF / EXPERT_GEMM_GU_ROWS);
+        const long grid = (sw.n_cu + 7) / 8 * 8, items = (long)((N + 63) / 64) * (FF / EXPERT_GEMM_GU_ROWS);
         const double gu_us = 4.5 * (double)((items + grid - 1) / grid * (H / 256));
         if (!q6k_gemm_pays(gu_us + g.us + (ks > 1 ? 2.0 : 0.0), N,
                            [&] { return proj_chunks_us(FF, H, 2, N) + proj_chunks_us(H, FF, 1, N); }))

@@ -11,7 +11,6 @@ import pytest
 
 ROOT = Path(__file__).resolve().parent.parent
 GEMV, Q4K, Q80, F16, Q6K = range(5)
-N_CU = 256
 
 PROBE = r"""
 #include <cstdio>
@@ -26,7 +25,7 @@ int main() {
       printf("%%d 0 0\n", moe_gemm_pays(N, path, rows, K, true, force & 1, force < 2, 256));
       continue;
     }
-    const ProjRoute r = kind == 'p' ? proj_route(sw, path, rows, K, N, 256) : dense_route(sw, path, rows, K, N, 256);
+    const ProjRoute r = kind == 'p' ? proj_route(sw, path, rows, K, N) : dense_route(sw, path, rows, K, N);
     printf("%%d %%d %%d\n", r.few, r.gemm_ks, r.chunk);
   }
 }
